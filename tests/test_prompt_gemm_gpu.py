@@ -1,0 +1,55 @@
+"""The prompt GEMM (zg_gemv_device, Q4_K, 256 rows and more): workgroup
+shapes, K splits and ragged edges against float64 on the dequantised weight.
+
+The bound: a weight is q s - m with s, m and the difference each rounded to
+f16, an activation is rounded to f16; a rounding's rms is 2^-11 / sqrt(3) =
+2.8e-4 of its operand, q s and m are about 1.5 times the weight, and the
+errors are independent over K, so an output's error has an rms of at most
+2.8e-4 sqrt(1.5^2 + 1.5^2 + 1 + 1) = 7.2e-4 of the outputs' rms.  1e-3 bounds
+the 2-norm, and 6e-3 (8 of those) each of up to 17 million outputs."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from zerogravity_amd import _lib as L
+from zerogravity_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def kern():
+    from zerogravity_amd import regions as R
+    k = R.HipMatVecKernel(0)
+    yield k
+    k.ctx.close()
+
+
+# one tile and the 256-row threshold, M and N one past and one short of a
+# tile, three and four K splits and none, a whole chip of each shape
+@pytest.mark.parametrize("M,N,K", [(256, 31, 256), (257, 129, 768), (300, 127, 3072), (385, 260, 3328), (601, 2048, 6144),
+                                   (640, 1030, 3584), (511, 8224, 1024), (1025, 2049, 2048), (2048, 8224, 512),
+                                   (4100, 4097, 256)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_prompt_gemm_matches_float64(kern, M, N, K, norm):
+    rng = np.random.default_rng(M + N + K)
+    w = synth.random_q4_k(rng, N, K)
+    h = kern.register(700, f"prompt.{M}.{N}.{K}.{norm}", synth.Q4_K, K, N, w.reshape(-1))
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).cuda()
+    g = torch.from_numpy((1 + 0.1 * rng.standard_normal(K)).astype(np.float32)).cuda()
+    y = torch.full((M + 1, N), 7.0, device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(2):
+        kern.ctx.check(L.lib().zg_gemv_device(kern.ctx.h, h.h, x.data_ptr(), L.F32, M, g.data_ptr() if norm else None,
+                                              1e-6, y.data_ptr(), None))
+    torch.cuda.synchronize()
+    xr = x.double()
+    if norm:
+        xr = xr / torch.sqrt((xr * xr).mean(1, keepdim=True) + 1e-6) * g.double()
+    ref = xr @ torch.from_numpy(h.dequantize()).cuda().double().t().contiguous()
+    err, rms = y[:M].double() - ref, ref.square().mean().sqrt().item()
+    assert err.square().mean().sqrt().item() <= 1e-3 * rms
+    assert err.abs().max().item() <= 6e-3 * rms
+    assert bool((y[M] == 7.0).all())  # nothing past the last row
+    kern.release_source(700)

@@ -102,7 +102,8 @@ void free_weight(zg_weight* w) {
     if (w->dw.hdr) (void)hipFree(w->dw.hdr);
     if (w->dw.qs_t) (void)hipFree(w->dw.qs_t);
     if (w->dw.hdr_t) (void)hipFree(w->dw.hdr_t);
-    w->dw.qs = w->dw.hdr = w->dw.qs_t = w->dw.hdr_t = nullptr;
+    if (w->dw.wh) (void)hipFree(w->dw.wh);
+    w->dw.qs = w->dw.hdr = w->dw.qs_t = w->dw.hdr_t = w->dw.wh = nullptr;
 }
 
 bool supported_type(int t) { return t == ZG_Q8_0 || t == ZG_Q4_K || t == ZG_F32 || t == ZG_Q4_1 || t == ZG_Q6_K; }
@@ -523,16 +524,26 @@ int zg_gemv_device(zg_ctx* ctx, const zg_weight* w, const void* x, int x_dtype, 
         f.ldy = w->dw.N;
         f.status = ctx->d_flag;
         if (device_batched(w, m_rows, pro)) {
-            // Q4_K: the 32-row weight tiles, unless the 16-row kernel takes this shape
-            if (w->dw.type == zg::kQ4_K && !w->dw.qs_t &&
-                !zg::batched16_supported(m_rows, w->dw.K, w->dw.N, zg::EPI_STORE)) {
+            // Q4_K: a prompt's f16 weight tiles, or the 32-row tiles unless the
+            // 16-row kernel takes this shape
+            const bool prompt = w->dw.type == zg::kQ4_K && m_rows >= (size_t)zg::kGemmRows;
+            if (prompt && !w->dw.wh) {
+                ZG_HIP(hipStreamSynchronize(s));
+                ZG_HIP(zg::ensure_f16_tiles(const_cast<zg_weight*>(w)->dw, s));
+            } else if (!prompt && w->dw.type == zg::kQ4_K && !w->dw.qs_t &&
+                       !zg::batched16_supported(m_rows, w->dw.K, w->dw.N, zg::EPI_STORE)) {
                 ZG_HIP(hipStreamSynchronize(s));
                 ZG_HIP(zg::ensure_mfma_tiles(const_cast<zg_weight*>(w)->dw, s));
             }
-            const size_t need = zg::batched_scratch_bytes(m_rows, w->dw.K);
+            // a prompt's partial sums behind its activation tiles
+            const size_t act = align256(zg::batched_scratch_bytes(m_rows, w->dw.K));
+            const int splits = prompt ? zg::prompt_splits(m_rows, w->dw.K, w->dw.N) : 1;
+            f.prompt_parts_n = splits > 1 ? (size_t)splits * m_rows * w->dw.N : 0;
+            const size_t need = act + f.prompt_parts_n * sizeof(float);
             if (ctx->actbuf.bytes < need) ZG_HIP(hipStreamSynchronize(s));
             int rc = ensure(ctx, ctx->actbuf, need);
             if (rc) return rc;
+            if (f.prompt_parts_n) f.prompt_parts = (float*)((char*)ctx->actbuf.ptr + act);
             ZG_HIP(zg::batched_gemv(w->dw, f, ctx->actbuf.ptr, s));
         } else {
             ZG_HIP(zg::fused_gemv(w->dw, f, s));

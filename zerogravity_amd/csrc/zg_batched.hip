@@ -808,7 +808,12 @@ hipError_t batched_gemv(const DeviceWeight& w, const FusedGemvArgs& args, void* 
     if (w.type != kQ4_K || w.K % 256 || w.K > 8192 || args.M <= 0 || args.M > 65535 * 32) return hipErrorInvalidValue;
     if (args.pro == PRO_GATED && args.group != 128) return hipErrorInvalidValue;
     const bool m16 = batched16_supported((size_t)args.M, w.K, w.N, args.epi);
-    if (!m16 && (!w.qs_t || !w.hdr_t)) return hipErrorNotReady;  // ensure_mfma_tiles first
+    // prompt-sized M: the f16 GEMM (zg_gemm.hip); a pending split-K or RMS
+    // tiles belong to the decode step's 32-row kernel
+    const bool prompt = args.M >= kGemmRows && !(args.epi == EPI_RESID && args.splits > 1 && args.parts) &&
+                        !args.rms_tiles_out && !args.rms_ss_in && prompt_gemm_supported(w.type, w.K, w.N, args.epi);
+    // ensure_f16_tiles / ensure_mfma_tiles first
+    if (prompt ? !w.wh : !m16 && (!w.qs_t || !w.hdr_t)) return hipErrorNotReady;
     FusedGemvArgs a = args;
     a.qs = m16 ? w.qs : w.qs_t;  // the 16-row kernel reads the Q4_K tile layout itself
     a.hdr = m16 ? w.hdr : w.hdr_t;
@@ -841,11 +846,7 @@ hipError_t batched_gemv(const DeviceWeight& w, const FusedGemvArgs& args, void* 
     }
     if ((a.rms_tiles_out || a.rms_ss_in) && a.splits > 1) return hipErrorInvalidValue;
     if (a.rms_ss_in && a.rms_ss_n > 64) return hipErrorInvalidValue;  // 8 sums per thread, 8+ threads per row
-    // prompt-sized M: the register-blocked GEMM (zg_gemm.hip)
-    const bool no_split = !(a.epi == EPI_RESID && a.splits > 1 && a.parts);
-    if (a.M >= kGemmRows && no_split && !a.rms_tiles_out && !a.rms_ss_in &&
-        prompt_gemm_supported(w.type, w.K, w.N, a.epi))
-        return prompt_gemm(w, args, xh, s);
+    if (prompt) return prompt_gemm(w, args, xh, s);
     if (a.epi == EPI_GLU) {
         if (!batched_glu_supported(w.type, w.K, w.N) || !a.xh_out) return hipErrorInvalidValue;
         dim3 g((unsigned)(a.N / 64), (unsigned)(mpad / 32), 1u);

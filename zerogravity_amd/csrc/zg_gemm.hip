@@ -1,19 +1,24 @@
 // Prompt-sized projections (M >= kGemmRows rows): Y[m][n] (+)= sum_k X[m][k] W[n][k]
 // with X the f16 activation tiles act16_kernel writes and W the Q4_K weight
-// in MFMA tile order (ensure_mfma_tiles), dequantized in registers.
+// dequantized once to f16 tiles of the same order (ensure_f16_tiles).
 //
-// Register-blocked on v_mfma_f32_32x32x16_f16: a workgroup of 4 waves, WN
-// along N and 4/WN along M; each wave owns MT x NT output tiles of 32 x 32
-// (MT*NT*16 accumulators).  The K loop walks 64-wide steps: the
-// workgroup's AT = (4/WN)*MT activation tiles of a step (AT x 4 KB) are
-// staged in LDS (two buffers, the next step's loads in flight during the
-// MFMAs), each wave loads its NT weight tiles' nibbles (one 16-byte load
-// per lane per tile) and dequantizes them once per step, so every
-// dequantized B fragment feeds MT MFMAs and every A fragment read from LDS
-// feeds NT.  The dequantization and the operand layouts are those of
-// mfma_q4k_kernel (the decode path's batched GEMM); its f16 rounding of the
-// weights and f32 accumulation make the result agree with the CPU's f32
-// dot within the per-op tolerance.
+// gemm_f16_kernel: v_mfma_f32_32x32x16_f16 on operands staged in LDS by
+// direct buffer_load ... lds copies.  Both operands lie in memory as 1 KB
+// fragments (32 rows x 16 columns, the 64 lanes' 16-byte words in lane
+// order), so a fragment is one wave instruction from memory to LDS and one
+// conflict-free ds_read_b128 from LDS to registers.  A workgroup of 8 waves
+// owns (MT WM) x (NT WN) tiles of 32 x 32, each wave MT x NT; ST stages of
+// 32 columns rotate in LDS, ST - 1 of them in flight while one is
+// multiplied, and each wave reads the next 16 columns' fragments before the
+// current ones' products, across the stage barrier too.
+//
+// What bounds it: power.  At M = 2048, N = 12288, K = 2048 the GEMM alone
+// runs 101 us = 1021 TFLOP/s on random operands and 78 us = 1318 TFLOP/s on
+// zeros (same instructions), the library's f16 product 106 us.  The kernel
+// this replaces dequantized the weights in every workgroup (5 VALU
+// operations per two weights before each operand's products): 135 us for
+// the same projection.  The f16 copy costs N K 2 bytes per weight; reading
+// four times the bytes of the codec's own payload is hidden from 256 rows on.
 #include <algorithm>
 
 #include "zg_decode_common.hpp"
@@ -27,215 +32,257 @@ typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 
 constexpr float kF16Max = 65504.0f;
+constexpr int kFrags = 2;  // 16-column fragments per tile and stage
 
-// Element (m, k) of the f16 A tiles for K columns: the act16_kernel layout.
-__device__ __forceinline__ size_t a_tile_index(int m, int k, int K) {
-    return ((((size_t)(m >> 5) * (K >> 8) + (k >> 8)) * 16 + ((k & 255) >> 4)) * 64 + ((k & 15) >> 3) * 32 +
-            (m & 31)) * 8 + (k & 7);
+}  // namespace
+
+// One 1 KB fragment from memory into LDS: lane l's 16 bytes at byte
+// `offset` + 16 l of a strip of `bytes` bytes go to `lds` + 16 l.
+__device__ __forceinline__ void copy_frag(const _Float16* strip, int bytes, int offset, int lane, char* lds) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)strip, 0, bytes, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, lane * 16, offset, 0,
+                                             0);
 }
 
-template <int EPI, int MT, int NT, int WN, int WM>
-__global__ __launch_bounds__(64 * WN * WM, 1) void gemm_q4k_kernel(FusedGemvArgs a, const _Float16* __restrict__ xh) {
-    constexpr int AT = WM * MT, NTHR = 64 * WN * WM, APT = AT * 256 / NTHR;  // A slabs per thread
-    static_assert(EPI != EPI_GLU || NT % 2 == 0, "SwiGLU pairs gate and up tiles");
-    static_assert(AT * 256 % NTHR == 0, "whole activation slabs per thread");
-    __shared__ h8v xs[2][AT * 256];  // AT tiles x 4 steps x 64 lanes of 16 bytes
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, hsel = lane >> 5, r32 = lane & 31;
+// up * silu(gate) of values the fast form covers (|gate| < 80: the exponent
+// stays in range, so ggml_exp's scaling branches and its finite check drop
+// out and its bits stay); the quotient by a reciprocal with one Newton step
+// and one residual correction instead of the scaled division.  The 16 values
+// of a lane's tile in ggml_silu took about 50 VALU instructions each, 19 us
+// of the 2048 x 12288 projection's 124.
+__device__ __forceinline__ float silu_product(float g, float up) {
+    const float x = 0.0f - g, r = __uint_as_float(0x4b400000u);
+    const float z = fmaf(x, __uint_as_float(0x3fb8aa3bu), r), n = z - r;
+    const float b = fmaf(-n, __uint_as_float(0x35bfbe8eu), fmaf(-n, __uint_as_float(0x3f317200u), x));
+    const float k = __uint_as_float((__float_as_uint(z) << 23) + 0x3f800000u), u = b * b;
+    const float j = fmaf(fmaf(fmaf(__uint_as_float(0x3c072010u), b, __uint_as_float(0x3d2b9f17u)), u,
+                              fmaf(__uint_as_float(0x3e2aaf33u), b, __uint_as_float(0x3efffedbu))),
+                         u, __uint_as_float(0x3f7ffff6u) * b);
+    const float d = 1.0f + fmaf(j, k, k);
+    float y = __builtin_amdgcn_rcpf(d);
+    y = fmaf(fmaf(-d, y, 1.0f), y, y);
+    float q = g * y;
+    q = fmaf(fmaf(-q, d, g), y, q);
+    return up * q;
+}
+
+// Grid of mg x ng x S tiles in one dimension, 64 WM WN threads.  Workgroups go
+// round-robin to the 8 XCDs: each XCD takes a contiguous run of the tile
+// order (bands of 8 tiles along M, M fastest), so its L2 holds the operands
+// its 32 CUs share.  S > 1: run z of the K columns into parts[z].
+template <int EPI, int MT, int NT, int WM, int WN, int ST>
+__global__ __launch_bounds__(64 * WM * WN, 1) void gemm_f16_kernel(FusedGemvArgs a, const _Float16* __restrict__ xh,
+                                                                   const _Float16* __restrict__ wh, int mg, int ng) {
+    constexpr int W = WM * WN, TA = MT * WM, TB = NT * WN, FR = (TA + TB) * kFrags, LPW = FR / W;
+    static_assert(FR % W == 0 && NT == 2, "whole loads per wave; a wave's two weight tiles are a SwiGLU pair");
+    __shared__ __attribute__((aligned(16))) char lds[ST][FR * 1024];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wv / WN, wn = wv - wm * WN;
-    const int K = a.K, N = a.N, nbk = K >> 8;
-    // split-K (residual projections with splits > 1): workgroup z takes the
-    // z-th of S equal runs of 256-column blocks and writes its partial tile
-    const int S = EPI == EPI_RESID && a.splits > 1 ? a.splits : 1, z = blockIdx.z;
-    const int blk0 = z * nbk / S, blk1 = (z + 1) * nbk / S;
-    const int nsub = 4 * blk1;  // one past this run's last 64-column step
-    const int mtiles = (a.M + 31) >> 5;
-    const int mt0 = blockIdx.y * AT;
+    const int S = EPI != EPI_GLU && a.splits > 1 ? a.splits : 1;
+    const int total = mg * ng * S, xc = blockIdx.x & 7, li = blockIdx.x >> 3;
+    const int per = total >> 3, rem = total & 7, lt = xc * per + min(xc, rem) + li;
+    const int z = lt / (mg * ng), t = lt - z * mg * ng;
+    const int band = t / (8 * ng), bw = min(8, mg - 8 * band), tb = t - band * 8 * ng;
+    const int bm = 8 * band + tb % bw, bn = tb / bw;
+    const int N = a.N, kf = a.K >> 4, mtiles = (a.M + 31) >> 5, ntiles = (N + 31) >> 5;
+    // stage s covers fragments kFrags s ..; this run's stages [s0, s0 + ns)
+    const int s0 = z * (kf / kFrags) / S, ns = (z + 1) * (kf / kFrags) / S - s0;
 
-    // this wave's weight tiles; with SwiGLU the first NT/2 are gate tiles and
-    // the rest the up tiles N/64 later (rows j and N/2 + j pair up)
-    constexpr int NW = EPI == EPI_GLU ? NT / 2 : NT;
-    const int wtile0 = (blockIdx.x * WN + wn) * NW;
-    int nbase[NT];
-    bool nv[NT];
-    uint32_t qoff[NT], hoff[NT];  // byte offsets of this lane's weight / header runs
+    // Weight tile of slot b of this workgroup: wave wn's slots are 2 wn and
+    // 2 wn + 1; with SwiGLU slot 2 wn is a gate tile and 2 wn + 1 the up tile
+    // N/64 tiles later (rows j and N/2 + j pair up).
+    auto wtile = [&](int b) { return EPI == EPI_GLU ? bn * (TB / 2) + (b >> 1) + (b & 1) * (N >> 6) : bn * TB + b; };
+    // the K strip of each of this wave's loads (tiles past the end read the
+    // last one; their results are dropped)
+    const _Float16* strip[LPW];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const int tile = EPI == EPI_GLU ? (t < NW ? wtile0 + t : wtile0 + t - NW + (N >> 6)) : wtile0 + t;
-        nbase[t] = tile * 32;
-        nv[t] = EPI == EPI_GLU ? (wtile0 + (t % NW)) * 32 + r32 < (N >> 1) : nbase[t] + r32 < N;
-        const int tt = min(tile, (N - 1) >> 5);  // tiles past the end read the last one (results dropped)
-        qoff[t] = ((uint32_t)tt * nbk * 256 + lane) * 16;
-        hoff[t] = ((uint32_t)tt * nbk * 32 + r32) * 16;
+    for (int i = 0; i < LPW; ++i) {
+        const int f = wv + i * W, tile = f / kFrags;
+        strip[i] = tile < TA ? xh + (size_t)min(bm * TA + tile, mtiles - 1) * kf * 512
+                             : wh + (size_t)min(wtile(tile - TA), ntiles - 1) * kf * 512;
     }
-    // buffer resources sized to each operand (32-bit byte offsets: the host
-    // refuses an operand of 4 GiB or more, prompt_gemm_bytes)
-    const uint32_t ntl = (uint32_t)((N + 31) >> 5);
-    const __amdgpu_buffer_rsrc_t rq =
-        __builtin_amdgcn_make_buffer_rsrc((void*)a.qs, 0, (int)(ntl * (uint32_t)nbk * 4096u), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rh =
-        __builtin_amdgcn_make_buffer_rsrc((void*)a.hdr, 0, (int)(ntl * (uint32_t)nbk * 512u), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rx =
-        __builtin_amdgcn_make_buffer_rsrc((void*)xh, 0, (int)((uint32_t)mtiles * (uint32_t)K * 64u), 0x00020000);
-    // slab e (of AT*256) of a step: tile e/256, h8v e%256 of its 4-step run
-    uint32_t aoff[APT];
+    auto load = [&](int s, int buf) {
 #pragma unroll
-    for (int i = 0; i < APT; ++i) {
-        const int e = tid + i * NTHR;
-        const int mt = min(mt0 + e / 256, mtiles - 1);  // tiles past the end read the last one (results dropped)
-        aoff[i] = ((uint32_t)mt * nbk * 16 * 64 + (e & 255)) * 16;
-    }
-
-    // Weights two steps ahead in a two-slot ring (slot = step parity), the
-    // activation slab and the next block's headers one step / one block
-    // ahead.  Requests past the end re-read the last step or block, so every
-    // path issues the same loads and the compiler's load counting never
-    // waits on a later request.  (Measured at the 2B shapes against one
-    // step ahead: L=8192 model prefill 1% faster, L=2048 unchanged.)
-    h8v ast[APT];
-    v4u wq[2][NT], hc[NT], hn[NT];
-    auto load_a = [&](int sb) {
-        sb = min(sb, nsub - 1);
-        const uint32_t astep = (uint32_t)((sb >> 2) * 16 + 4 * (sb & 3)) * 64 * 16;
-#pragma unroll
-        for (int i = 0; i < APT; ++i)
-            ast[i] = __builtin_bit_cast(h8v, __builtin_amdgcn_raw_buffer_load_b128(rx, aoff[i] + astep, 0, 0));
+        for (int i = 0; i < LPW; ++i) {
+            const int f = wv + i * W;
+            copy_frag(strip[i], kf * 1024, ((s0 + s) * kFrags + f % kFrags) * 1024, lane, &lds[buf][f * 1024]);
+        }
     };
-    auto load_w = [&](int sb, v4u (&dst)[NT]) {
-        sb = min(sb, nsub - 1);
+    h8v fa[2][MT], fb[2][NT];
+    auto frags = [&](int buf, int k, int slot) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t) dst[t] = __builtin_amdgcn_raw_buffer_load_b128(rq, qoff[t] + (uint32_t)sb * 64 * 16, 0, 0);
-    };
-    auto load_h = [&](int blk, v4u (&dst)[NT]) {
-        blk = min(blk, blk1 - 1);
+        for (int i = 0; i < MT; ++i)
+            fa[slot][i] = *(const h8v*)&lds[buf][(((wm * MT + i) * kFrags + k) * 64 + lane) * 16];
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
-            dst[t] = __builtin_amdgcn_raw_buffer_load_b128(rh, hoff[t] + (uint32_t)blk * 32 * 16, 0, 0);
+        for (int j = 0; j < NT; ++j)
+            fb[slot][j] = *(const h8v*)&lds[buf][(((TA + wn * NT + j) * kFrags + k) * 64 + lane) * 16];
     };
-    auto store = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < APT; ++i) xs[buf][tid + i * NTHR] = ast[i];
-    };
-
     f16v acc[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[i][t] = f16v{};
+        for (int j = 0; j < NT; ++j) acc[i][j] = f16v{};
 
-    load_a(4 * blk0);
-    load_h(blk0, hc);
-    load_w(4 * blk0, wq[0]);
-    load_w(4 * blk0 + 1, wq[1]);
-    store(0);
-    __syncthreads();
-    const h2v bias = h2v{(_Float16)1024.0f, (_Float16)1024.0f};
-    for (int blk = blk0; blk < blk1; ++blk) {
-        load_h(blk + 1, hn);
+    // K >= 256 gives ns >= 2 stages per run (K >= 3072 with splits), ST - 1 <= 3
 #pragma unroll
-        for (int c4 = 0; c4 < 4; ++c4) {
-            const int sb = 4 * blk + c4, cur = c4 & 1;
-            load_a(sb + 1);
-            // the two 32-groups of this step: scale and min rounded once to f16
-            h2v sc[NT][2], nm[NT][2];
+    for (int s = 0; s < ST - 1; ++s) load(min(s, ns - 1), s);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LPW * (ST - 2)) : "memory");
+    frags(0, 0, 0);
+    load(min(ST - 1, ns - 1), ST - 1);
+    for (int sb = 0; sb < ns; sb += ST) {
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const float d = f16_to_f32((uint16_t)(hc[t].x & 0xffffu));
-                const float dmin = f16_to_f32((uint16_t)(hc[t].x >> 16));
+        for (int u = 0; u < ST; ++u) {
+            const int s = sb + u;
+            if (s >= ns) break;
+            frags(u, 1, 1);
+            __builtin_amdgcn_sched_barrier(0);  // the reads go out before the products they overlap
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    uint32_t s, mn;
-                    q4k_dev_scale_min(hc[t], 2 * c4 + h, s, mn);
-                    const _Float16 sh = (_Float16)(d * (float)s), mh = (_Float16)(dmin * (float)mn);
-                    sc[t][h] = h2v{sh, sh};
-                    nm[t][h] = h2v{-mh, -mh};
-                }
-            }
-            // each weight dword's low and high nibbles, masked once per step:
-            // step j takes dwords (2 (j%2), 2 (j%2) + 1), low nibbles for j < 2
-            uint32_t nib[NT][2][4];
+            for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const uint32_t wd[4] = {wq[cur][t].x, wq[cur][t].y, wq[cur][t].z, wq[cur][t].w};
+                for (int i = 0; i < MT; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[0][i], fb[0][j], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            // stage s + 1 has landed (each wave waits for its own copies, the
+            // barrier for the others'), and every wave has read stage s, whose
+            // buffer then takes stage s + ST.  Every pass issues the same
+            // LPW copies (past the end: the last stage again), so the count
+            // left in flight is a constant.
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LPW * (ST - 2)) : "memory");
+            frags((u + 1) % ST, 0, 0);
+            load(min(s + ST, ns - 1), u);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    nib[t][0][q] = wd[q] & 0x0f0f0f0fu;
-                    nib[t][1][q] = (wd[q] >> 4) & 0x0f0f0f0fu;
-                }
-            }
-            load_w(sb + 2, wq[cur]);  // the slot is free once its nibbles are out
+            for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                h8v af[MT];
-#pragma unroll
-                for (int i = 0; i < MT; ++i) af[i] = xs[cur][(wm * MT + i) * 256 + j * 64 + lane];
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    // step j: nibble half j/2 of the 8-byte piece j%2 (group 2*c4 + j/2)
-                    const uint32_t w0 = nib[t][j >> 1][2 * (j & 1)], w1 = nib[t][j >> 1][2 * (j & 1) + 1];
-                    // bytes (q, 0x64) pairs: the f16 bit patterns of 1024 + q
-                    const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, w0, 0x04010400u);
-                    const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, w0, 0x04030402u);
-                    const uint32_t p2 = __builtin_amdgcn_perm(0x64646464u, w1, 0x04010400u);
-                    const uint32_t p3 = __builtin_amdgcn_perm(0x64646464u, w1, 0x04030402u);
-                    const h2v s2 = sc[t][j >> 1], n2 = nm[t][j >> 1];
-                    const h2v e0 = __builtin_elementwise_fma(__builtin_bit_cast(h2v, p0) - bias, s2, n2);
-                    const h2v e1 = __builtin_elementwise_fma(__builtin_bit_cast(h2v, p1) - bias, s2, n2);
-                    const h2v e2 = __builtin_elementwise_fma(__builtin_bit_cast(h2v, p2) - bias, s2, n2);
-                    const h2v e3 = __builtin_elementwise_fma(__builtin_bit_cast(h2v, p3) - bias, s2, n2);
-                    // (a tile past N computes on a clamped copy; its columns are never stored)
-                    const h8v wb = h8v{e0[0], e0[1], e1[0], e1[1], e2[0], e2[1], e3[0], e3[1]};
-#pragma unroll
-                    for (int i = 0; i < MT; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], wb, acc[i][t], 0, 0, 0);
-                }
-            }
-            store(cur ^ 1);  // (past the last step: a copy of it into the idle buffer)
-            __syncthreads();
+                for (int i = 0; i < MT; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[1][i], fb[1][j], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int t = 0; t < NT; ++t) hc[t] = hn[t];
     }
+    // no copy into LDS outlives its use below, or the workgroup
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
-    // D register r of tile (i, t) is row (r%4) + 8*(r/4) + 4*(lane/32) of the
+    // D register r of tile (i, j) is row (r%4) + 8*(r/4) + 4*(lane/32) of the
     // activation tile, column lane%32 of the weight tile
+    const int hsel = lane >> 5, r32 = lane & 31;
     bool over = false;
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-        const int tile_m = mt0 + wm * MT + i;
-        if (tile_m >= mtiles) continue;
+        const int tm = bm * TA + wm * MT + i;
+        if (tm >= mtiles) continue;
+        if constexpr (EPI == EPI_GLU) {
+            // up * silu(gate) in f32, rounded once to f16 into the down
+            // projection's A tiles (K = N/2 columns); a value past the f16
+            // range raises status bit 4.  The 32 x 32 products are two of
+            // those fragments: turned in the wave's own LDS (2 KB), stored as
+            // whole 16-byte words.
+            _Float16* turn = (_Float16*)lds + wv * 1024;
+            bool small = true;  // (false for a NaN gate)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m = tile_m * 32 + (r & 3) + 8 * (r >> 2) + 4 * hsel;
-            if (EPI == EPI_GLU) {
+            for (int r = 0; r < 16; ++r) small &= fabsf(acc[i][0][r]) < 80.0f;
+            const bool fast = __all(small);
 #pragma unroll
-                for (int t = 0; t < NW; ++t) {
-                    if (!nv[t]) continue;
-                    // up * silu(gate) in f32, rounded once to f16 into the down
-                    // projection's A tiles (K = N/2 columns); a value past the
-                    // f16 range raises status bit 4
-                    const float v = m < a.M ? acc[i][t + NW][r] * ggml_silu(acc[i][t][r]) : 0.0f;
-                    over |= !(fabsf(v) <= kF16Max);
-                    ((_Float16*)a.xh_out)[a_tile_index(m, nbase[t] + r32, N >> 1)] = (_Float16)v;
-                }
-            } else {
+            for (int r = 0; r < 16; ++r) {
+                const int m32 = (r & 3) + 8 * (r >> 2) + 4 * hsel;
+                float v = fast ? silu_product(acc[i][0][r], acc[i][1][r]) : acc[i][1][r] * ggml_silu(acc[i][0][r]);
+                if (tm * 32 + m32 >= a.M) v = 0.0f;
+                over |= !(fabsf(v) <= kF16Max);
+                turn[((r32 >> 4) * 64 + ((r32 & 15) >> 3) * 32 + m32) * 8 + (r32 & 7)] = (_Float16)v;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            const h8v o0 = *(const h8v*)(turn + lane * 8), o1 = *(const h8v*)(turn + 512 + lane * 8);
+            _Float16* dst = (_Float16*)a.xh_out + ((size_t)tm * (N >> 5) + 2 * (bn * (TB / 2) + wn)) * 512;
+            *(h8v*)(dst + lane * 8) = o0;
+            *(h8v*)(dst + 512 + lane * 8) = o1;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // both words read before the next tile turns
+        } else {
+            const int m0 = tm * 32 + 4 * hsel, n0 = (bn * TB + wn * NT) * 32 + r32;
+            auto row = [](int r) { return (r & 3) + 8 * (r >> 2); };
+            // the residual rows are all requested before the first is used
+            // (read and written element by element, each add waited on a
+            // load: 35 us of a 2048 x 2048 x 2048 projection, 21 without)
+            float old[EPI == EPI_RESID ? 16 : 1][NT];
+            if constexpr (EPI == EPI_RESID) {
 #pragma unroll
-                for (int t = 0; t < NT; ++t)
-                    if (nv[t] && m < a.M) {
-                        if (S > 1)
-                            a.parts[((size_t)z * a.M + m) * N + nbase[t] + r32] = acc[i][t][r];
-                        else
-                            epilogue(a, m, nbase[t] + r32, acc[i][t][r], EPI);
+                for (int r = 0; r < 16; ++r)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        old[r][j] = m0 + row(r) < a.M && n0 + 32 * j < N
+                                        ? a.y[(size_t)(m0 + row(r)) * a.ldy + n0 + 32 * j]
+                                        : 0.0f;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + row(r);
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    const int n = n0 + 32 * j;
+                    if (m >= a.M || n >= N) continue;
+                    if constexpr (EPI == EPI_RESID) {
+                        const float v = old[r][j] + acc[i][j][r];
+                        over |= !finite_f32(v);
+                        a.y[(size_t)m * a.ldy + n] = v;
+                    } else if (S > 1) {
+                        a.parts[((size_t)z * a.M + m) * N + n] = acc[i][j][r];
+                    } else {
+                        a.y[(size_t)m * a.ldy + n] = acc[i][j][r];
                     }
+                }
             }
         }
     }
-    if (EPI == EPI_GLU && over && a.status) atomicOr(a.status, 16);
+    // SwiGLU: past the f16 range; residual: nonfinite
+    if (over && a.status) atomicOr(a.status, EPI == EPI_GLU ? 16 : 1);
 }
 
-// y[m][n] += (parts[0] + parts[1]) (+ parts[2] + parts[3]) at (m, n), the
-// splits summed in order, float4 per thread; a non-finite sum raises status
-// bit 1 as the residual epilogue does.
-template <int S>
-__global__ __launch_bounds__(256) void split_resid_kernel(FusedGemvArgs a) {
+// Grid (tiles, K/256), 256 threads: columns 256 kb.. of the 32 rows of tile
+// `tile`, dequantized to f16 fragments.  Thread (c4, lane) holds row lane%32,
+// columns 64 c4 + 32 half + 16 piece + 8 (lane/32) .. +7 of the four
+// fragments (half, piece); scale and min of a 32-group rounded once to f16,
+// the weight q s - m as one f16 fma.  Rows past N are zero.
+__global__ __launch_bounds__(256) void f16_tile_q4k_kernel(const uint8_t* __restrict__ qs, const v4u* __restrict__ hdr,
+                                                           int N, int K, _Float16* __restrict__ wh) {
+    const int tile = blockIdx.x, kb = blockIdx.y, nbk = K >> 8;
+    const int c4 = threadIdx.x >> 6, lane = threadIdx.x & 63, row = tile * 32 + (lane & 31);
+    uint2 p[2] = {};
+    v4u hd = v4u{0u, 0u, 0u, 0u};
+    if (row < N) {
+        const uint8_t* b = qs + q4k_chunk_offset(row, 4 * kb + c4, K) + 8 * (lane >> 5);
+        p[0] = *(const uint2*)b;
+        p[1] = *(const uint2*)(b + 256);
+        hd = hdr[q4k_hdr_index(row, kb, nbk)];
+    }
+    const float d = f16_to_f32((uint16_t)(hd.x & 0xffffu)), dmin = f16_to_f32((uint16_t)(hd.x >> 16));
+    const h2v bias = h2v{(_Float16)1024.0f, (_Float16)1024.0f};
+    _Float16* dst = wh + (((size_t)tile * (K >> 4) + 16 * kb + 4 * c4) * 64 + lane) * 8;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        uint32_t s, mn;
+        q4k_dev_scale_min(hd, 2 * c4 + h, s, mn);
+        const _Float16 sh = (_Float16)(d * (float)s), mh = (_Float16)(dmin * (float)mn);
+        const h2v s2 = h2v{sh, sh}, n2 = h2v{-mh, -mh};
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const uint32_t w0 = (p[q].x >> (4 * h)) & 0x0f0f0f0fu, w1 = (p[q].y >> (4 * h)) & 0x0f0f0f0fu;
+            h8v o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                // bytes (q, 0x64) pairs: the f16 bit patterns of 1024 + q
+                const uint32_t pr = __builtin_amdgcn_perm(0x64646464u, e < 2 ? w0 : w1, e & 1 ? 0x04030402u : 0x04010400u);
+                const h2v v = __builtin_elementwise_fma(__builtin_bit_cast(h2v, pr) - bias, s2, n2);
+                o[2 * e] = v[0];
+                o[2 * e + 1] = v[1];
+            }
+            *(h8v*)(dst + (size_t)(2 * h + q) * 512) = o;
+        }
+    }
+}
+
+// y[m][n] (+)= (parts[0] + parts[1]) (+ parts[2]) (+ parts[3]) at (m, n), the
+// splits summed in order, float4 per thread; with ADD (residual) a
+// non-finite sum raises status bit 1 as the residual epilogue does.
+template <int S, bool ADD>
+__global__ __launch_bounds__(256) void split_sum_kernel(FusedGemvArgs a) {
     const size_t i4 = (size_t)blockIdx.x * 256 + threadIdx.x, n4 = (size_t)a.M * a.N / 4;
     if (i4 >= n4) return;
     const size_t e = 4 * i4, m = e / a.N, n = e % a.N, mn = (size_t)a.M * a.N;
@@ -243,26 +290,84 @@ __global__ __launch_bounds__(256) void split_resid_kernel(FusedGemvArgs a) {
 #pragma unroll
     for (int z = 0; z < S; ++z) p[z] = *(const v4f*)(a.parts + z * mn + e);
     float* yp = a.y + m * a.ldy + n;
-    const v4f y = *(const v4f*)yp;
-    v4f r;
+    v4f r = ADD ? *(const v4f*)yp : v4f{0.0f, 0.0f, 0.0f, 0.0f};
     bool bad = false;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         float acc = p[0][q];
 #pragma unroll
         for (int z = 1; z < S; ++z) acc = acc + p[z][q];
-        r[q] = y[q] + acc;
+        r[q] = ADD ? r[q] + acc : acc;
         bad |= !finite_f32(r[q]);
     }
     *(v4f*)yp = r;
-    if (bad) atomicOr(a.status, 1);
+    if (ADD && bad) atomicOr(a.status, 1);
+}
+
+namespace {
+
+// Workgroup shapes, rows x columns: 256 x 256 (one per CU: 128 KB of LDS),
+// 128 x 256 and 128 x 128 (two per CU).
+enum { SHAPE_256x256, SHAPE_128x256, SHAPE_128x128 };
+
+long tiles_of(size_t n, size_t w) { return (long)((n + w - 1) / w); }
+
+// The shape with the least time by measured rates: full chips of workgroups
+// (512, or 256 of 256 x 256) and the tail by its size.  In us at K = 2048,
+// the weights read from HBM as a model's are: 256 workgroups of 256 x 256
+// 66 (64 alone: 45), 512 of 128 x 256 70 (256: 36, 64: 26), 512 of
+// 128 x 128 44 (256: 19-21, 64: 13); with the weights in the Infinity Cache
+// the 128-wide shapes are 67 and 38, which moves no choice by more than 5%.
+int choose_shape(size_t M, size_t N) {
+    const long l = tiles_of(M, 256) * tiles_of(N, 256), b = tiles_of(M, 128) * tiles_of(N, 256),
+               c = tiles_of(M, 128) * tiles_of(N, 128);
+    auto tail = [](long r, double few, double some, double many) {
+        return r == 0 ? 0.0 : r <= 64 ? few : r <= 256 ? some : many;
+    };
+    const double tl = (l / 256) * 66.0 + tail(l % 256, 45.0, 62.0, 62.0);
+    const double tb = (b / 512) * 70.0 + tail(b % 512, 26.0, 36.0, 70.0);
+    const double tc = (c / 512) * 44.0 + tail(c % 512, 13.5, 19.0, 44.0);
+    return tc <= tb && tc <= tl ? SHAPE_128x128 : tb <= tl ? SHAPE_128x256 : SHAPE_256x256;
+}
+
+template <int EPI>
+hipError_t launch_gemm(const FusedGemvArgs& a, int shape, const _Float16* xh, const _Float16* wh, hipStream_t s) {
+    const int S = EPI != EPI_GLU && a.splits > 1 ? a.splits : 1;
+    const int mg = (int)tiles_of(a.M, shape == SHAPE_256x256 ? 256 : 128);
+    const int ng = (int)tiles_of(a.N, shape == SHAPE_128x128 ? 128 : 256);
+    const dim3 g((unsigned)(mg * ng * S));
+    if (shape == SHAPE_256x256)
+        hipLaunchKernelGGL((gemm_f16_kernel<EPI, 4, 2, 2, 4, 4>), g, dim3(512), 0, s, a, xh, wh, mg, ng);
+    else if (shape == SHAPE_128x256)
+        hipLaunchKernelGGL((gemm_f16_kernel<EPI, 2, 2, 2, 4, 3>), g, dim3(512), 0, s, a, xh, wh, mg, ng);
+    else
+        hipLaunchKernelGGL((gemm_f16_kernel<EPI, 1, 2, 4, 2, 4>), g, dim3(512), 0, s, a, xh, wh, mg, ng);
+    return hipGetLastError();
 }
 
 }  // namespace
 
-// Largest operand of the prompt GEMM in bytes: the f16 activation tiles
-// (32 rows x K per tile), the 32-row weight tiles and their headers.  Every
-// one must stay below 4 GiB (32-bit buffer offsets).
+hipError_t ensure_f16_tiles(DeviceWeight& w, hipStream_t s) {
+    if (w.type != kQ4_K || w.K % 256 || w.N == 0) return hipErrorInvalidValue;
+    if (w.wh) return hipSuccess;
+    const size_t tiles = (w.N + 31) / 32;
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, tiles * w.K * 64);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(f16_tile_q4k_kernel, dim3((unsigned)tiles, (unsigned)(w.K / 256)), dim3(256), 0, s,
+                       (const uint8_t*)w.qs, (const v4u*)w.hdr, (int)w.N, (int)w.K, (_Float16*)p);
+    e = hipGetLastError();
+    if (e != hipSuccess) {
+        (void)hipFree(p);
+        return e;
+    }
+    w.wh = p;
+    return hipSuccess;
+}
+
+// Largest operand of the prompt GEMM in bytes: the f16 activation tiles (32
+// rows x K per tile) and the codec's own 32-row tiles and headers.  A prompt
+// at 4 GiB or more of any is refused.
 uint64_t prompt_gemm_bytes(size_t M, size_t K, size_t N) {
     const uint64_t mt = (M + 31) / 32, nt = (N + 31) / 32, nbk = K / 256;
     return std::max({mt * K * 64, nt * nbk * 4096, nt * nbk * 512});
@@ -274,72 +379,40 @@ bool prompt_gemm_supported(int type, size_t K, size_t N, int epi) {
     return true;
 }
 
-// Shapes: two weight tiles per wave (NT = 2), four waves along N, and the
-// most activation tiles per wave (MT = 3, 2, 1) that still gives at least one
-// workgroup per CU (256), else one.  Measured over M = 512, 2048, 8192 and
-// the 2B-shaped projections (gate/up 12288 x 2048, GDN in 8224 x 2048, out
-// 2048 x 2048, down 2048 x 6144): NT = 4 tiles with MT = 4 left a
-// workgroup's 256 accumulators to one wave per SIMD and ran 1.3-1.6x
-// slower (gate/up at M = 2048: 176 against 127 us); with NT = 2 the choice
-// among MT = 1-4 and 2-8 waves moves the time by about 10%.
+// K splits: 128 x 128 tiles that fill at most half the CUs, with K long
+// enough that the shorter runs outweigh the second launch (M = 601, N = 2048,
+// K = 6144: 36 us unsplit, 21 us in three runs plus about 5 us for the sum;
+// M = 1024: 39 us, 29 us in two).  At most 256 tiles of partial sums, 4 Mi floats.
+int prompt_splits(size_t M, size_t K, size_t N) {
+    const long c = tiles_of(M, 128) * tiles_of(N, 128);
+    return K >= 3072 && N % 4 == 0 && c <= 128 ? (int)std::min<long>(4, 256 / c) : 1;
+}
+
 hipError_t prompt_gemm(const DeviceWeight& w, const FusedGemvArgs& args, const _Float16* xh, hipStream_t s) {
-    if (!prompt_gemm_supported(w.type, w.K, w.N, args.epi) || !w.qs_t || !w.hdr_t || args.M <= 0)
-        return hipErrorInvalidValue;
+    if (!prompt_gemm_supported(w.type, w.K, w.N, args.epi) || !w.wh || args.M <= 0) return hipErrorInvalidValue;
     if (args.epi == EPI_GLU && !args.xh_out) return hipErrorInvalidValue;
     if (prompt_gemm_bytes((size_t)args.M, w.K, w.N) >= ((uint64_t)1 << 32)) return hipErrorInvalidValue;
     FusedGemvArgs a = args;
-    a.qs = w.qs_t;
-    a.hdr = w.hdr_t;
     a.K = (int)w.K;
     a.N = (int)w.N;
-    const int mtiles = (a.M + 31) / 32;
-    const int ntiles = a.epi == EPI_GLU ? a.N / 64 : (a.N + 31) / 32;  // SwiGLU: gate/up tile pairs
-    auto grid = [&](int mt, int nt, int wn, int wm) {
-        const int nw = a.epi == EPI_GLU ? nt / 2 : nt;
-        return dim3((unsigned)((ntiles + wn * nw - 1) / (wn * nw)), (unsigned)((mtiles + wm * mt - 1) / (wm * mt)));
-    };
-    auto count = [&](dim3 g) { return (long)g.x * g.y; };
-#define ZG_GQ(E, MTV, NTV, WNV, WMV)                                                                                   \
-    hipLaunchKernelGGL((gemm_q4k_kernel<E, MTV, NTV, WNV, WMV>), grid(MTV, NTV, WNV, WMV), dim3(64 * WNV * WMV), 0, s, \
-                       a, xh)
-#define ZG_GQE(E)                                                  \
-    if (count(grid(3, 2, 4, 1)) >= 256) ZG_GQ(E, 3, 2, 4, 1);      \
-    else if (count(grid(2, 2, 4, 1)) >= 256) ZG_GQ(E, 2, 2, 4, 1); \
-    else ZG_GQ(E, 1, 2, 4, 1);
-    // residual projections whose tiles give fewer than one 4-wave workgroup
-    // per CU (or exactly one, for K >= 4096) split K in two or four runs of
-    // 256-column blocks, and a second launch adds the runs into y: measured
-    // at the 2B shapes, L=512 model prefill 7.58 -> 6.31 ms (four-way splits
-    // where the tiles give at most 64 workgroups), L=2048 14.46 -> 14.28 ms
-    const long c2 = count(grid(2, 2, 4, 1));
-    int S = 1;
-    if (a.epi == EPI_RESID && a.prompt_parts && a.N % 4 == 0 && a.ldy % 4 == 0) {
-        if (c2 <= 64 && (a.K / 256) % 4 == 0) S = 4;
-        else if ((c2 < 256 || (c2 == 256 && a.K >= 4096)) && (a.K / 256) % 2 == 0) S = 2;
-    }
-    if (S > 1 && (size_t)S * a.M * a.N > a.prompt_parts_n) S = 1;
+    a.splits = 0;
+    const _Float16* wh = (const _Float16*)w.wh;
+    if (a.epi == EPI_GLU) return launch_gemm<EPI_GLU>(a, choose_shape(a.M, a.N), xh, wh, s);
+    int S = a.prompt_parts && a.ldy % 4 == 0 && (uintptr_t)a.y % 16 == 0 ? prompt_splits(a.M, w.K, w.N) : 1;
+    if ((size_t)S * a.M * a.N > a.prompt_parts_n) S = 1;
     if (S > 1) {
         a.splits = S;
         a.parts = a.prompt_parts;
-        dim3 g = grid(2, 2, 4, 1);
-        g.z = (unsigned)S;
-        hipLaunchKernelGGL((gemm_q4k_kernel<EPI_RESID, 2, 2, 4, 1>), g, dim3(256), 0, s, a, xh);
-        const size_t n4 = (size_t)a.M * a.N / 4;
-        if (S == 4) hipLaunchKernelGGL(split_resid_kernel<4>, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, a);
-        else hipLaunchKernelGGL(split_resid_kernel<2>, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, a);
+        const hipError_t e = launch_gemm<EPI_STORE>(a, SHAPE_128x128, xh, wh, s);
+        if (e != hipSuccess) return e;
+        const dim3 g((unsigned)(((size_t)a.M * a.N / 4 + 255) / 256));
+#define ZG_SUM(SV)                                                                                                 if (a.epi == EPI_RESID) hipLaunchKernelGGL((split_sum_kernel<SV, true>), g, dim3(256), 0, s, a);               else hipLaunchKernelGGL((split_sum_kernel<SV, false>), g, dim3(256), 0, s, a);
+        if (S == 4) { ZG_SUM(4) } else if (S == 3) { ZG_SUM(3) } else { ZG_SUM(2) }
+#undef ZG_SUM
         return hipGetLastError();
     }
-    a.splits = 0;
-    if (a.epi == EPI_GLU) {
-        ZG_GQE(EPI_GLU)
-    } else if (a.epi == EPI_RESID) {
-        ZG_GQE(EPI_RESID)
-    } else {
-        ZG_GQE(EPI_STORE)
-    }
-#undef ZG_GQE
-#undef ZG_GQ
-    return hipGetLastError();
+    const int shape = choose_shape(a.M, a.N);
+    return a.epi == EPI_RESID ? launch_gemm<EPI_RESID>(a, shape, xh, wh, s) : launch_gemm<EPI_STORE>(a, shape, xh, wh, s);
 }
 
 }  // namespace zg

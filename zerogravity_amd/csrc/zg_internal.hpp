@@ -32,6 +32,9 @@ struct DeviceWeight {
     // headers in the MFMA operand order of 32-row tiles (ensure_mfma_tiles).
     void* qs_t = nullptr;
     void* hdr_t = nullptr;
+    // Q4_K only, built on demand for prompts: the weight dequantized to f16
+    // MFMA tiles (ensure_f16_tiles), N rounded up to 32 rows.
+    void* wh = nullptr;
 };
 
 size_t gguf_row_bytes(int type, size_t K);
@@ -44,8 +47,8 @@ hipError_t repack_weight(const uint8_t* d_gguf, DeviceWeight& w, int* d_bad, hip
 // f32 [rows][K].
 hipError_t dequantize_rows(const DeviceWeight& w, size_t row0, size_t rows, float* out, hipStream_t s);
 
-// Activation rows from which batched_gemv runs the register-blocked prompt
-// GEMM (zg_gemm.hip) instead of the decode-shaped MFMA kernel.
+// Activation rows from which batched_gemv runs the prompt GEMM (zg_gemm.hip)
+// instead of the decode-shaped MFMA kernels.
 constexpr int kGemmRows = 256;
 
 // f16 activation tiles of the batched GEMMs, element (m, k) for K columns.
@@ -200,10 +203,10 @@ struct FusedGemvArgs {
     int splits = 0;
     const float* rparts = nullptr;
     int rsplits = 0;
-    // prompt-sized residual projections (optional): workspace of
-    // prompt_parts_n floats for the prompt GEMM's own split over K (two or
-    // four runs of S x M x N partial sums), summed into y by a second launch
-    // in a fixed order; a split that would not fit is not taken
+    // prompt-sized projections (optional): workspace of prompt_parts_n floats
+    // for the prompt GEMM's own split over K (prompt_splits runs of M x N
+    // partial sums), summed into y by a second launch in a fixed order; a
+    // split that would not fit is not taken
     float* prompt_parts = nullptr;
     size_t prompt_parts_n = 0;
     float* xw = nullptr;
@@ -276,6 +279,9 @@ size_t batched_scratch_bytes(size_t M, size_t K);
 // Builds w.qs_t / w.hdr_t (Q4_K) if absent: allocates, so call it outside
 // graph capture.  batched_gemv refuses a Q4_K weight without them.
 hipError_t ensure_mfma_tiles(DeviceWeight& w, hipStream_t s);
+// Builds w.wh (Q4_K) if absent, likewise: batched_gemv refuses a prompt
+// (M >= kGemmRows) without it.
+hipError_t ensure_f16_tiles(DeviceWeight& w, hipStream_t s);
 hipError_t batched_gemv(const DeviceWeight& w, const FusedGemvArgs& a, void* scratch, hipStream_t s);
 // Q8_0 beyond 4 rows (zg_q8rows.hip): every activation row coded once into
 // `scratch` in act_prepare_for's layout (prepared_bytes(kQ8_0, M, K), within
@@ -298,6 +304,9 @@ hipError_t q8_rows_prepared(const DeviceWeight& w, size_t M, const void* prepare
 bool prompt_gemm_supported(int type, size_t K, size_t N, int epi);
 hipError_t prompt_gemm(const DeviceWeight& w, const FusedGemvArgs& a, const _Float16* xh, hipStream_t s);
 uint64_t prompt_gemm_bytes(size_t M, size_t K, size_t N);
+// Runs over K the prompt GEMM takes when given a workspace (prompt_parts) of
+// that many M x N partial sums; 1: none.
+int prompt_splits(size_t M, size_t K, size_t N);
 
 // GDN decode: conv (4-slot ring per channel) + SiLU + q/k L2 + gates +
 // recurrence for B rows.  proj rows: [qkv (3W) | z (W) | alpha (H) | beta (H)].

@@ -1273,7 +1273,8 @@ int prefill_batched_body(zg_session* s, size_t row, size_t n, const uint32_t* to
     int rc0 = sync_positions(s, st);
     if (rc0) return rc0;
     for (zg_weight* w : ws)
-        if (!w->dw.qs_t) ZG_HIP(zg::ensure_mfma_tiles(w->dw, st));
+        if (n >= (size_t)zg::kGemmRows) ZG_HIP(zg::ensure_f16_tiles(w->dw, st));
+        else if (!zg::xh16_layout(n, w->dw.K)) ZG_HIP(zg::ensure_mfma_tiles(w->dw, st));
     const size_t H = g.hidden, F = g.ffn, W = (size_t)g.gdn_heads * g.gdn_dim, GH = g.gdn_heads;
     const size_t QD = (size_t)g.q_heads * g.head_dim;
     const size_t mpad = (n + 31) / 32 * 32;
@@ -1284,10 +1285,9 @@ int prefill_batched_body(zg_session* s, size_t row, size_t n, const uint32_t* to
             return fail(ctx, ZG_E_LIMIT, "prompt too long for the batched prefill (an operand of its projections "
                                          "would reach 4 GiB): split it over several calls");
     enum { X, P, Q, K, V, BETA, LOGD, CORE, QB, OB, XH, XH2, CHUNK, TOK, ATTP, RPARTS, NBUF };
-    // the split residual projections' partial sums: a split is taken only
-    // while the tiles give at most 256 workgroups of 64 x 256 outputs, so two
-    // runs of those (or four of a quarter as many) bound it
-    const size_t kSplitParts = 2 * 256 * 64 * 256;
+    // the split residual projections' partial sums: splits times tiles stay
+    // within 256 workgroups of 128 x 128 outputs (prompt_splits)
+    const size_t kSplitParts = 256 * 128 * 128;
     if (n > s->pf_cap) {
         ZG_HIP(hipStreamSynchronize(st));
         for (void* p : s->pf) (void)hipFree(p);
