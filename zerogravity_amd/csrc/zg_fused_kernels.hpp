@@ -298,6 +298,108 @@ __global__ __launch_bounds__(256) void fused_q8_kernel(FusedGemvArgs a) {
 }
 
 
+// Narrow Q8_0 projections (few 8-row groups): one 8-row group per workgroup,
+// its four waves splitting K.  The integer dots of a row are independent;
+// only the reference's chain of K/32 fused multiply-adds per lane is serial.
+// So each wave requests all of its chunks at once (CW of four blocks), forms
+// its blocks' dots and scales, and the waves then run the chain one after
+// another, handing the accumulators on through LDS: the same products in the
+// same order, bit for bit, on four times the waves.
+// What bounds it: launch, prologue and one memory round trip.  Against
+// fused_q8_kernel, whose waves take a group each (us, one row, N x K):
+// 1024 x 3584 9.4 -> 5.4 (32 -> 128 workgroups), 2048 x 6144 13.9 -> 9.2,
+// 1024 x 2048 5.8 -> 3.8; four rows 22.2 -> 8.3, 33.4 -> 19.4, 13.3 -> 8.6.
+template <int MT, int J, int CW, int PRO, int EPI>
+__global__ __launch_bounds__(256) void fused_q8_relay_kernel(FusedGemvArgs a) {
+    // CW chunks per wave: 4 CW blocks of 4 cover K <= 512 CW
+    extern __shared__ int lds_r8[];
+    __shared__ float relay[3][MT][64];
+    const int K = a.K, N = a.N;
+    const int nb = K >> 5, nbc = (nb + 3) >> 2, nbp = nbc * 4, nbs = nbp + 4;
+    int* codes = lds_r8;                               // [MT][8][nbs] words (wg_prologue's Q8_0 layout)
+    float* scales = (float*)(lds_r8 + MT * 8 * nbs);   // [MT][nbp]
+    const int m0 = blockIdx.y * MT;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rl = lane >> 3, l = lane & 7;
+    const int R = blockIdx.x, row = R * 8 + rl, rowc = min(row, N - 1);
+    const int c0 = wv * nbc / 4, c1 = (wv + 1) * nbc / 4;  // this wave's chunks, at most CW
+    ProIn<J> pin;
+    wg_prologue_load<PRO, J>(a, m0, m0 < a.M, pin);
+    v4i w[CW];
+    uint2 h[CW];
+    {
+        const v4i* tile = (const v4i*)a.qs + (size_t)R * nbc * 64 + lane;
+        const uint16_t* hrow = (const uint16_t*)a.hdr + (size_t)rowc * nbc * 4;
+#pragma unroll
+        for (int i = 0; i < CW; ++i) {
+            const int c = min(c0 + i, nbc - 1);
+            w[i] = load_nt(tile + (size_t)c * 64);
+            h[i] = *(const uint2*)(hrow + 4 * c);
+        }
+    }
+    float old[MT];  // the residual outputs, requested ahead of the chain
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+        old[m] = EPI == EPI_RESID && wv == 3 && m0 + m < a.M ? a.y[(size_t)(m0 + m) * a.ldy + rowc] : 0.0f;
+    wg_prologue_code<PRO, kCodecQ8, J>(a, m0 < a.M, pin, nullptr, codes, scales);
+#pragma unroll
+    for (int m = 1; m < MT; ++m)
+        wg_prologue<PRO, kCodecQ8, J>(a, m0 + m, m0 + m < a.M, nullptr, codes + (size_t)m * 8 * nbs,
+                                      scales + (size_t)m * nbp);
+    float p[MT][4 * CW], sc[MT][4 * CW];
+#pragma unroll
+    for (int i = 0; i < CW; ++i) {
+        const int c = min(c0 + i, nbc - 1);
+        const bool in = c0 + i < c1;
+        const int ww[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
+        const uint32_t hw[4] = {h[i].x & 0xffffu, h[i].x >> 16, h[i].y & 0xffffu, h[i].y >> 16};
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const v4i cw = *(const v4i*)(codes + (size_t)(m * 8 + l) * nbs + 4 * c);
+            const v4f sw = *(const v4f*)(scales + (size_t)m * nbp + 4 * c);
+#pragma unroll
+            for (int bi = 0; bi < 4; ++bi) {
+                // a block past the wave's range or the row's end adds 0 * 0:
+                // the accumulator, never -0, keeps its bits
+                const bool ok = in && 4 * c + bi < nb;
+                const float pair = (float)__builtin_amdgcn_sdot4(ww[bi], cw[bi], 0, false);
+                const float scale = f16_to_f32((uint16_t)hw[bi]) * sw[bi];
+                p[m][4 * i + bi] = ok ? pair : 0.0f;
+                sc[m][4 * i + bi] = ok ? scale : 0.0f;
+            }
+        }
+    }
+    float acc[MT];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        if (wv == t) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[m] = t == 0 ? 0.0f : relay[t > 0 ? t - 1 : 0][m][lane];
+#pragma unroll
+            for (int i = 0; i < 4 * CW; ++i)
+#pragma unroll
+                for (int m = 0; m < MT; ++m) acc[m] = fmaf(p[m][i], sc[m][i], acc[m]);
+            if (t < 3) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m) relay[t][m][lane] = acc[m];
+            }
+        }
+        if (t < 3) lds_barrier();
+    }
+    if (wv != 3) return;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[m] = group8_tree_last(acc[m]);  // the reference's lane tree, in lane 7
+    if (row < N && l == 7) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            if (m0 + m >= a.M) continue;
+            const float v = EPI == EPI_RESID ? old[m] + acc[m] : acc[m];
+            a.y[(size_t)(m0 + m) * a.ldy + row] = v;
+            if (EPI == EPI_RESID && !finite_f32(v)) atomicOr(a.status, 1);
+        }
+    }
+}
+
 // ====================================================== Q4_1, Q6_K, F32
 
 // Q4_1 x Q8_1 (cpu/src/source/quantization.rs:198-227): lane l of a row's 8
@@ -734,6 +836,37 @@ hipError_t launch_q8(const FusedGemvArgs& a, hipStream_t s) {
     // codes 8 words per block (rows padded by 4 words) + a scale per block
     auto lds = [&](int t) { return (size_t)t * (8 * ((K / 32 + 3) / 4 * 4 + 4) + (K / 32 + 3) / 4 * 4) * 4; };
     const size_t groups = (a.N + 7) / 8;
+    // few row groups: K over a workgroup's waves (fused_q8_relay_kernel).
+    // Beyond these counts a wave per group fills the chip by itself and the
+    // relay's repeated prologue costs more: 7168 x 1024 one row 4.8 -> 4.6 us,
+    // two rows 6.3 -> 6.5; 12288 x 2048 one row even, two 11.3 -> 13.3.  (At
+    // long K a lane's products of two or four rows do not fit its registers:
+    // those rows go to further workgroups.)
+    if (groups <= (a.M == 1 ? 1152 : 512)) {
+        const int cw = K <= 1024 ? 2 : K <= 2048 ? 4 : K <= 4096 ? 8 : K <= 6144 ? 12 : 16;
+        while (mt * cw > 16) mt >>= 1;
+        const dim3 gr((unsigned)groups, (unsigned)((a.M + mt - 1) / mt));
+#define ZG_R8(T, JJ, C) hipLaunchKernelGGL((fused_q8_relay_kernel<T, JJ, C, PRO, EPI>), gr, dim3(256), lds(T), s, a)
+#define ZG_R8M(JJ, C)                  \
+    if (mt == 1) ZG_R8(1, JJ, C);      \
+    else if (mt == 2) ZG_R8(2, JJ, C); \
+    else ZG_R8(4, JJ, C);
+        if (cw == 2) {
+            ZG_R8M(1, 2)
+        } else if (cw == 4) {
+            ZG_R8M(2, 4)
+        } else if (cw == 8) {
+            if (mt == 1) ZG_R8(1, 4, 8);
+            else ZG_R8(2, 4, 8);
+        } else if (cw == 12) {
+            ZG_R8(1, 8, 12);
+        } else {
+            ZG_R8(1, 8, 16);
+        }
+#undef ZG_R8M
+#undef ZG_R8
+        return hipGetLastError();
+    }
     const unsigned wgs = (unsigned)std::min<size_t>((groups + 3) / 4, 256 * 8);
     dim3 g(wgs, (unsigned)((a.M + mt - 1) / mt));
 #define ZG_F8(T, JJ) hipLaunchKernelGGL((fused_q8_kernel<T, JJ, PRO, EPI>), g, dim3(256), lds(T), s, a)
