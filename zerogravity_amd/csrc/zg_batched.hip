@@ -820,7 +820,8 @@ hipError_t batched_gemv(const DeviceWeight& w, const FusedGemvArgs& args, void* 
     a.K = (int)w.K;
     a.N = (int)w.N;
     if (m16) {  // no split-K; the sums of squares fit 8 per thread
-        if ((a.epi == EPI_RESID && a.splits > 1 && a.parts) || (a.rms_ss_in && a.rms_ss_n > 128) ||
+        const bool small = small_batch_fits((size_t)a.M, w.K, w.N, a.epi);  // (checks its own count of sums)
+        if ((a.epi == EPI_RESID && a.splits > 1 && a.parts) || (!small && a.rms_ss_in && a.rms_ss_n > 128) ||
             (a.rms_tiles_out && (a.epi != EPI_RESID || a.N % 128)) || (a.epi == EPI_GLU && !a.xh_out))
             return hipErrorInvalidValue;
     }
@@ -837,6 +838,7 @@ hipError_t batched_gemv(const DeviceWeight& w, const FusedGemvArgs& args, void* 
         default: return hipErrorInvalidValue;
         }
     }
+    if (m16 && small_batch_fits((size_t)a.M, w.K, w.N, a.epi)) return launch_small_batch(a, xh, s);
     if (m16) {
         switch (a.epi) {
         case EPI_GLU: return launch_mfma16<EPI_GLU>(a, xh, s);

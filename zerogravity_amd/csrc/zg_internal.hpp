@@ -214,7 +214,7 @@ struct FusedGemvArgs {
     // rms_tiles_out it also leaves the next RMS projection's input -- f16
     // (x_new * rms_gamma) in MFMA A-tile order for K = N (xh_tile_index),
     // and per row and 32-column tile (16-column on the 16-row kernel) the
-    // f64 sum of the f32 squares of x_new at rms_ss_out[m][N/32 or N/16].
+    // f64 sum of the f32 squares of x_new at rms_ss_out[m][N/rms_ss_columns].
     // That RMS projection passes the tiles as xh_in and the sums as
     // rms_ss_in (rms_ss_n per row) and scales each row's outputs by 1/rms
     // (RMSNorm's factor moved past the dot).
@@ -262,6 +262,12 @@ int batched_splits(size_t N, size_t K);
 // (no split-K; xh16_layout(M, K) holds, and a residual projection with
 // rms_tiles_out leaves rms_ss_out[m][N/16]).
 bool batched16_supported(size_t M, size_t K, size_t N, int epi);
+// 2..8 rows of such a shape take the small-batch kernel (zg_small_batch.hip).
+bool small_batch_fits(size_t M, size_t K, size_t N, int epi);
+hipError_t launch_small_batch(const FusedGemvArgs& a, const void* xh, hipStream_t s);
+// Columns per sum of squares a batched residual projection of this shape
+// leaves in rms_ss_out (its tile width).
+int rms_ss_columns(size_t M, size_t K, size_t N);
 bool fused_gemv_supported(int type, size_t K, size_t N, int pro);
 // Greedy partials the one-row matrix-core GEMV leaves for this weight with
 // EPI_STORE (0 when the weight takes another kernel).

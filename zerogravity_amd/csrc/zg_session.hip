@@ -420,7 +420,7 @@ int step(zg_session* s, size_t B, const uint32_t* tokens, float* logits, uint32_
                 const bool h16 = zg::xh16_layout(B, H);
                 rms_ready = gamma_next && H % 256 == 0 && H <= 2048 && ldy == H &&
                             (h16 ? k16 : !k16 && w->dw.K <= 2048);
-                rss_n = (int)(k16 ? H / 16 : H / 32);
+                rss_n = (int)(H / zg::rms_ss_columns(B, w->dw.K, H));
                 const int sp = rms_ready || k16 ? 1 : zg::batched_splits(w->dw.N, w->dw.K);
                 if (rms_ready) {
                     f.rms_tiles_out = (_Float16*)s->xh3;
