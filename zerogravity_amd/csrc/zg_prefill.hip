@@ -48,10 +48,16 @@ typedef float f4m __attribute__((ext_vector_type(4)));
 // Record per (chunk, head), floats.  W first holds the solve's right-hand
 // side (beta k) exp(g); U is overwritten in place by corr in the scan; A is
 // the decayed (beta k) k^T (strictly lower part used); S holds the state
-// entering the chunk, key-major [k][v].
+// entering the chunk, key-major [k][v].  The solved W and dk are stored in
+// the scan's operand order, so that a lane reads its MFMA operands of four
+// steps as one 16-byte word: W row t holds column k at perm_w(k); dk is
+// [key d][64], token t at perm_t(t).
 constexpr size_t kOffU = 0, kOffW = kOffU + kC * kD, kOffDq = kOffW + kC * kD, kOffDk = kOffDq + kC * kD,
                  kOffIntra = kOffDk + kC * kD, kOffA = kOffIntra + kC * kC, kOffDecay = kOffA + kC * kC,
                  kOffS = kOffDecay + 64, kRec = kOffS + kD * kD;
+
+__device__ __forceinline__ int perm_w(int k) { return 32 * (k & 3) + (k >> 2); }
+__device__ __forceinline__ int perm_t(int t) { return 16 * (t & 3) + (t >> 2); }
 
 __device__ __forceinline__ f4m mfma4(float a, float b, f4m c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -206,8 +212,19 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const float* __rest
         const int f = tid + 256 * i, t = f >> 5, d = 4 * (f & 31);
         const v4f qv = *(const v4f*)&qs[t * kPad + d], kv = *(const v4f*)&ks[t * kPad + d];
         *(v4f*)(rec + kOffDq + t * kD + d) = qv * eg[t];
-        *(v4f*)(rec + kOffDk + t * kD + d) = kv * el[t];
         *(v4f*)(rec + kOffW + t * kD + d) = (kv * bs[t]) * eg[t];
+    }
+    // dk in the scan's order: word (key d, four steps from t = 16 s4 + kq)
+#pragma unroll
+    for (int i = 0; i < kC * kD / 4 / 256; ++i) {
+        const int f = tid + 256 * i, d = f >> 4, kq = (f >> 2) & 3, s4 = f & 3;
+        v4f o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = 4 * (4 * s4 + e) + kq;
+            o[e] = ks[t * kPad + d] * el[t];
+        }
+        *(v4f*)(rec + kOffDk + d * kC + 16 * kq + 4 * s4) = o;
     }
     if (tid < 64) rec[kOffDecay + tid] = cr_expf(gs[kC - 1]);  // replicated for vector loads
 }
@@ -277,31 +294,41 @@ __global__ __launch_bounds__(128) void gdn_chunk_solve_kernel(const float* __res
         // hoisted further, the reads held most of A in registers
         if (row >= 1) asm volatile("" ::"v"(xr[row - 1]) : "memory");
     }
-    float* dst = rec + (z == 0 ? kOffU : kOffW);
+    // W replaces its right-hand side in another column order: every column
+    // has been read
+    if (z != 0) __syncthreads();
+    float* dst = rec + (z == 0 ? kOffU + col : kOffW + perm_w(col));
 #pragma unroll
-    for (int t = 0; t < kC; ++t) dst[t * kD + col] = xr[t];
+    for (int t = 0; t < kC; ++t) dst[t * kD] = xr[t];
 }
 
 // Grid (H, kD / kSW), 512 threads: value columns [16 slab, 16 slab + 16) of
 // head h through all chunks in order (every slab of a head on one XCD, whose
-// L2 then serves the shared W and dk).  The state is held key-major S[k][j]
-// in LDS; in memory it is value-major [h][v][k] (the decode layout) or, with
-// key_major, [h][k][v] (the chunk reference's layout).  Per chunk the four
-// compute waves store the entering state, form pred = W S, corr = U - pred
-// (written over U), then S <- dk^T corr + exp(g_last) S, reading W, dk, the
-// U slab and the decay from LDS.  The four loader waves stage those: at
-// chunk c they write chunk c + 1's operands (requested two chunks earlier,
-// held in registers) into the LDS buffer chunk c - 1 used while the compute
-// waves form corr, and request chunk c + 3's while they update the state,
-// so no compute wave waits on global memory.  (Measured at 8192 tokens:
-// 2.9 us per chunk with the old one-wave-group form, whose end-of-chunk
-// wait covered the next chunk's loads and its own stores; 2.2 us here.)
+// L2 then serves the shared W and dk).  In memory the state is value-major
+// [h][v][k] (the decode layout) or, with key_major, [h][k][v] (the chunk
+// reference's layout).  Per chunk the four compute waves store the entering
+// state, form pred = W S, corr = U - pred (written over U), then
+// S <- dk^T corr + exp(g_last) S.  The four loader waves stage W, dk, the U
+// slab and the decay: at chunk c they write chunk c + 1's operands (requested
+// two chunks earlier, held in registers) into the LDS buffer chunk c - 1 used
+// while the compute waves form corr, and request chunk c + 3's while they
+// update the state, so no compute wave waits on global memory.
+//
+// What bounds it is the dependent chain of a chunk: 32 + 16 x 2 MFMAs (0.9
+// us) and, between them, the exchange of corr and of S through LDS and two
+// barriers.  So the state stays in its owner's MFMA registers (wave w: key
+// rows 32 w .. +31) and LDS holds only the copy the next product reads, every
+// operand in an order that four steps are one 16-byte read (40 LDS
+// instructions per wave and chunk instead of 140), and the operands that do
+// not depend on the state, W's and dk's, are read during the product before
+// theirs.  2048 tokens, 16 heads: 71 -> 59 us (1.85 us per chunk).
 __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(float* __restrict__ scratch, int T, int H,
                                                              float* __restrict__ state, int key_major) {
-    __shared__ float S[kD][kSW + 1];
-    __shared__ float Cr[kC][kSW + 1];
-    __shared__ float Wl[2][kC * kPad];
-    __shared__ float Dk[2][kC * kPad];
+    constexpr int kTpad = kC + 4;                 // row pitch of [..][64] operand rows
+    __shared__ float Sb[kSW * kPad];              // [column j][perm_w(key)]
+    __shared__ float Cr[kSW * kTpad];             // [column j][perm_t(token)]
+    __shared__ float Wl[2][kC * kPad];            // [token][perm_w(key)]
+    __shared__ float Dk[2][kD * kTpad];           // [key][perm_t(token)]
     __shared__ float Ub[2][kC][kSW];
     __shared__ float Dc[2];
     const int h = blockIdx.x, slab = blockIdx.y;
@@ -309,10 +336,6 @@ __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(float* __restrict__
     const bool loader = tid >= 256;
     const int j0 = slab * kSW, i0 = 16 * wv, jl = lane & 15, kq = lane >> 4;
     float* sh = state + (size_t)h * kD * kD;
-    for (int i = tid; i < kD * kSW; i += 512) {
-        const int kk = key_major ? i / kSW : i % kD, j = key_major ? i % kSW : i / kD;
-        S[kk][j] = key_major ? sh[(size_t)kk * kD + j0 + j] : sh[(size_t)(j0 + j) * kD + kk];
-    }
     const int nch = (T + kC - 1) / kC;
 
     // ---- loader waves: a chunk's operands in registers, then in LDS
@@ -324,9 +347,8 @@ __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(float* __restrict__
         const float* rec = scratch + ((size_t)c * H + h) * kRec;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const int f = lt + 256 * i;  // row f / 32, float4 f % 32
-            o.w[i] = *(const v4f*)(rec + kOffW + (f >> 5) * kD + 4 * (f & 31));
-            o.dk[i] = *(const v4f*)(rec + kOffDk + (f >> 5) * kD + 4 * (f & 31));
+            o.w[i] = *(const v4f*)(rec + kOffW + 4 * (lt + 256 * i));
+            o.dk[i] = *(const v4f*)(rec + kOffDk + 4 * (lt + 256 * i));
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -340,7 +362,7 @@ __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(float* __restrict__
         for (int i = 0; i < 8; ++i) {
             const int f = lt + 256 * i;
             *(v4f*)&Wl[buf][(f >> 5) * kPad + 4 * (f & 31)] = o.w[i];
-            *(v4f*)&Dk[buf][(f >> 5) * kPad + 4 * (f & 31)] = o.dk[i];
+            *(v4f*)&Dk[buf][(f >> 4) * kTpad + 4 * (f & 15)] = o.dk[i];
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -350,77 +372,77 @@ __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(float* __restrict__
         if (lt == 0) Dc[buf] = o.decay;
     };
 
-    // ---- compute waves: one chunk from LDS buffer buf
+    // ---- compute waves: registers of S (tile i: key rows 32 wv + 16 i + 4 kq
+    // + r, column jl), of W's operands and of dk's
+    f4m S[2];
+    v4f wa[kD / 16], da[2][kC / 16];
+    auto key_of = [&](int i, int r) { return 32 * wv + 16 * i + 4 * kq + r; };
+    auto publish = [&]() {  // S into LDS for the next W S
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) Sb[jl * kPad + perm_w(key_of(i, r))] = S[i][r];
+    };
+    auto read_w = [&](int buf) {
+#pragma unroll
+        for (int q = 0; q < kD / 16; ++q) wa[q] = *(const v4f*)&Wl[buf][(i0 + jl) * kPad + 32 * kq + 4 * q];
+    };
     auto step = [&](int c, int buf) {
         float* rec = scratch + ((size_t)c * H + h) * kRec;
+        v4f sb[kD / 16];
+#pragma unroll
+        for (int q = 0; q < kD / 16; ++q) sb[q] = *(const v4f*)&Sb[jl * kPad + 32 * kq + 4 * q];
+        float ub[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ub[r] = Ub[buf][i0 + 4 * kq + r][jl];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int q = 0; q < kC / 16; ++q)
+                da[i][q] = *(const v4f*)&Dk[buf][(32 * wv + 16 * i + jl) * kTpad + 16 * kq + 4 * q];
         // the state entering this chunk, for the output kernel
-        {
-            float sv[kD * kSW / 256];
 #pragma unroll
-            for (int i = 0; i < kD * kSW / 256; ++i) {
-                const int f = lt + 256 * i;
-                sv[i] = S[f / kSW][f % kSW];
-            }
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int i = 0; i < kD * kSW / 256; ++i) {
-                const int f = lt + 256 * i;
-                rec[kOffS + (f / kSW) * kD + j0 + f % kSW] = sv[i];
-            }
-        }
+            for (int r = 0; r < 4; ++r) rec[kOffS + key_of(i, r) * kD + j0 + jl] = S[i][r];
+        __builtin_amdgcn_sched_barrier(0);  // the reads go out before the chain
         // pred = W S: wave w owns rows 16w..16w+15
         f4m acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int s0 = 0; s0 < kD / 4; s0 += 16) {  // operand reads in two halves (registers)
-            float wa[16], sb[16];
+        for (int q = 0; q < kD / 16; ++q)
 #pragma unroll
-            for (int s = 0; s < 16; ++s) {
-                wa[s] = Wl[buf][(i0 + jl) * kPad + 4 * (s0 + s) + kq];
-                sb[s] = S[4 * (s0 + s) + kq][jl];
-            }
-            __builtin_amdgcn_sched_barrier(0);  // issue the half's operand reads before its chain
-#pragma unroll
-            for (int s = 0; s < 16; ++s) acc = mfma4(wa[s], sb[s], acc);
-        }
+            for (int e = 0; e < 4; ++e) acc = mfma4(wa[q][e], sb[q][e], acc);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int t = i0 + 4 * kq + r;
-            const float cr = Ub[buf][t][jl] - acc[r];
-            Cr[t][jl] = cr;
+            const float cr = ub[r] - acc[r];
+            Cr[jl * kTpad + perm_t(t)] = cr;
             rec[kOffU + t * kD + j0 + jl] = cr;
         }
     };
     auto update = [&](int buf) {
-        // S <- dk^T corr + decay S: wave w owns key rows 32w..32w+31
+        // S <- dk^T corr + decay S
         const float decay = Dc[buf];
+        v4f cb[kC / 16];
+#pragma unroll
+        for (int q = 0; q < kC / 16; ++q) cb[q] = *(const v4f*)&Cr[jl * kTpad + 16 * kq + 4 * q];
+        read_w(buf ^ 1);  // the next chunk's (staged before the last barrier; past the end unused)
+        __builtin_amdgcn_sched_barrier(0);
         f4m sn[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
-        float sold[2][4];
 #pragma unroll
-        for (int it2 = 0; it2 < 2; ++it2)
+        for (int q = 0; q < kC / 16; ++q)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) sold[it2][r] = S[32 * wv + 16 * it2 + 4 * kq + r][jl];
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int s0 = 0; s0 < kC / 4; s0 += 8) {
-            float cb[8], da[2][8];
+                for (int i = 0; i < 2; ++i) sn[i] = mfma4(da[i][q][e], cb[q][e], sn[i]);
 #pragma unroll
-            for (int s = 0; s < 8; ++s) {
-                const int tt = 4 * (s0 + s) + kq;
-                cb[s] = Cr[tt][jl];
-#pragma unroll
-                for (int it2 = 0; it2 < 2; ++it2) da[it2][s] = Dk[buf][tt * kPad + 32 * wv + 16 * it2 + jl];
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int s = 0; s < 8; ++s)
-#pragma unroll
-                for (int it2 = 0; it2 < 2; ++it2) sn[it2] = mfma4(da[it2][s], cb[s], sn[it2]);
-        }
-#pragma unroll
-        for (int it2 = 0; it2 < 2; ++it2)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float sd = sold[it2][r] * decay;
-                S[32 * wv + 16 * it2 + 4 * kq + r][jl] = sn[it2][r] + sd;
+                const float sd = S[i][r] * decay;
+                S[i][r] = sn[i][r] + sd;
             }
+        publish();
     };
 
     // The two groups run separate loops that meet at the same barriers (two
@@ -438,8 +460,8 @@ __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(float* __restrict__
         // staging overlaps the compute waves' first half (state store, W S,
         // corr), the next request their second (the state update)
         auto chunk = [&](int c, Ops& nxt) {
-            if (c + 1 < nch) stage((c + 1) & 1, nxt);
-            lds_barrier();  // chunk c + 1 staged
+            stage((c + 1) & 1, nxt);  // (past the last chunk: a copy of it, never used)
+            lds_barrier();            // chunk c + 1 staged
             fetch(min(c + 3, nch - 1), nxt);
             lds_barrier();
         };
@@ -450,20 +472,32 @@ __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(float* __restrict__
         }
         if (c < nch) chunk(c, rb);
     } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int k = key_of(i, r);
+                S[i][r] = key_major ? sh[(size_t)k * kD + j0 + jl] : sh[(size_t)(j0 + jl) * kD + k];
+            }
+        publish();
         __syncthreads();
+        read_w(0);
         for (int c = 0; c < nch; ++c) {
             step(c, c & 1);
             lds_barrier();  // corr visible to every compute wave
             update(c & 1);
             lds_barrier();  // S updated
         }
-    }
-    for (int i = tid; i < kD * kSW; i += 512) {
-        const int kk = key_major ? i / kSW : i % kD, j = key_major ? i % kSW : i / kD;
-        if (key_major)
-            sh[(size_t)kk * kD + j0 + j] = S[kk][j];
-        else
-            sh[(size_t)(j0 + j) * kD + kk] = S[kk][j];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int k = key_of(i, r);
+                if (key_major)
+                    sh[(size_t)k * kD + j0 + jl] = S[i][r];
+                else
+                    sh[(size_t)(j0 + jl) * kD + k] = S[i][r];
+            }
     }
 }
 
