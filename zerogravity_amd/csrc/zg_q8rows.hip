@@ -403,29 +403,40 @@ hipError_t launch_mfma_rows(const FusedGemvArgs& a, const int8_t* aq, const floa
     // R 16-row tiles per wave task while the waves stay plentiful
     const int R = tiles >= 2 * 4096 ? 2 : 1;
     const unsigned wgs = (unsigned)std::min<size_t>(((tiles + R - 1) / R + 3) / 4, 1024);
-    // MT activation rows per workgroup: as many as M needs up to 16, within
-    // 64 KB of LDS (two workgroups per CU), and fewer when the tiles alone
-    // would leave CUs idle (more workgroups along M, each re-reading the
-    // weights from cache)
-    int mt = 16;
-    while (mt > 4 && mt / 2 >= M) mt >>= 1;
-    while (mt > 4 && rows_lds(mt, K) > 65536) mt >>= 1;
-    while (mt > 4 && (size_t)wgs * ((M + mt - 1) / mt) < 256) mt >>= 1;
-    if (rows_lds(mt, K) > 65536) return hipErrorInvalidValue;
-    const unsigned gy = (unsigned)((M + mt - 1) / mt);
-    if (gy > 65535) return hipErrorInvalidValue;
-    const dim3 g(wgs, gy);
+    // Activation rows per workgroup: at most 16 within 64 KB of LDS (two
+    // workgroups per CU), the rows dealt evenly over as few workgroup rows as
+    // that allows -- more when the tiles alone would leave CUs idle (each
+    // re-reads the weights from cache) -- and rounded up to whole pairs: the
+    // padding rows cost what real ones do.  151936 x 2048 head, us: 11 rows
+    // as 16 134, as 12 114; 17 rows as 16 + 16 252, as 10 + 10 192; 33 rows
+    // 366, as 3 x 12 306.
+    int cap = 16;
+    while (cap > 4 && rows_lds(cap, K) > 65536) cap -= 2;
+    int gy = (M + cap - 1) / cap;
+    while ((size_t)wgs * gy < 256 && (M + gy - 1) / gy > 4) ++gy;
+    auto rows_of = [&](int y) { return std::max(4, ((M + y - 1) / y + 1) & ~1); };
+    // one workgroup row more where that pads less (16 rows as 4 x 4, not 3 x 6)
+    if ((size_t)wgs * gy < 512 && rows_of(gy) > 4 && rows_of(gy + 1) * (gy + 1) < rows_of(gy) * gy) ++gy;
+    const int mt = rows_of(gy);
+    gy = (M + mt - 1) / mt;
+    if (rows_lds(mt, K) > 65536 || gy > 65535) return hipErrorInvalidValue;
+    const dim3 g(wgs, (unsigned)gy);
     const size_t lds = rows_lds(mt, K);
 #define ZG_Q8M(MP_, R_) hipLaunchKernelGGL((q8_mfma_kernel<MP_, R_, EPI>), g, dim3(256), lds, s, a, aq, ad)
 #define ZG_Q8M_R(MP_)               \
-    if (R == 2) ZG_Q8M(MP_, 2);     \
-    else ZG_Q8M(MP_, 1);
-    if (mt == 16) {
-        ZG_Q8M_R(8)
-    } else if (mt == 8) {
-        ZG_Q8M_R(4)
-    } else {
+    case MP_:                       \
+        if (R == 2) ZG_Q8M(MP_, 2); \
+        else ZG_Q8M(MP_, 1);        \
+        break;
+    switch (mt / 2) {
         ZG_Q8M_R(2)
+        ZG_Q8M_R(3)
+        ZG_Q8M_R(4)
+        ZG_Q8M_R(5)
+        ZG_Q8M_R(6)
+        ZG_Q8M_R(7)
+        ZG_Q8M_R(8)
+    default: return hipErrorInvalidValue;
     }
 #undef ZG_Q8M_R
 #undef ZG_Q8M
