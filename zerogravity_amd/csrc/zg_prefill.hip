@@ -14,11 +14,11 @@
 //   o     =  intra corr + (q .* exp(g)) S
 //   S     <- (k .* exp(g_last - g))^T corr + exp(g_last) S
 //
-// Four launches.  gdn_chunk_prep_kernel runs every (chunk, head) in
+// Three launches.  gdn_chunk_prep_kernel runs every (chunk, head) in
 // parallel: normalisation, gates, A and intra on f32 MFMA (16x16x4), dq, dk
-// and exp(g_last), into a record per (chunk, head); gdn_chunk_solve_kernel
-// solves for U and W, one column per thread in the reference's summation
-// order.  gdn_chunk_scan_kernel carries the state through the chunks
+// and exp(g_last), into a record per (chunk, head), and the solves for U and
+// W, one column per thread in the reference's summation order.
+// gdn_chunk_scan_kernel carries the state through the chunks
 // in order, one workgroup per (head, 16-column value slab) since the value
 // columns of S evolve independently: per chunk only W S, corr = U - W S and
 // the state update, storing corr and the state entering the chunk.
@@ -45,15 +45,13 @@ constexpr int kPad = 132;                   // LDS row pitch (floats) of [rows][
 constexpr int kApad = 68;                   // LDS row pitch of [64][64] tiles
 typedef float f4m __attribute__((ext_vector_type(4)));
 
-// Record per (chunk, head), floats.  W first holds the solve's right-hand
-// side (beta k) exp(g); U is overwritten in place by corr in the scan; A is
-// the decayed (beta k) k^T (strictly lower part used); S holds the state
-// entering the chunk, key-major [k][v].  The solved W and dk are stored in
-// the scan's operand order, so that a lane reads its MFMA operands of four
+// Record per (chunk, head), floats.  U is overwritten in place by corr in the
+// scan; S holds the state entering the chunk, key-major [k][v].  W and dk are
+// stored in the scan's operand order, so that a lane reads its MFMA operands of four
 // steps as one 16-byte word: W row t holds column k at perm_w(k); dk is
 // [key d][64], token t at perm_t(t).
 constexpr size_t kOffU = 0, kOffW = kOffU + kC * kD, kOffDq = kOffW + kC * kD, kOffDk = kOffDq + kC * kD,
-                 kOffIntra = kOffDk + kC * kD, kOffA = kOffIntra + kC * kC, kOffDecay = kOffA + kC * kC,
+                 kOffIntra = kOffDk + kC * kD, kOffDecay = kOffIntra + kC * kC,
                  kOffS = kOffDecay + 64, kRec = kOffS + kD * kD;
 
 __device__ __forceinline__ int perm_w(int k) { return 32 * (k & 3) + (k >> 2); }
@@ -93,9 +91,20 @@ __device__ __forceinline__ void tile_pair(const float* Q, const float* K, int i0
 
 }  // namespace
 
-// Grid (chunks, H), 256 threads: everything of a (chunk, head) but the
-// solves.  LDS: q and k rows, 68 KB.
+// Grid (chunks, H), 256 threads: everything of a (chunk, head) but its place
+// in the sequence.  LDS: q and k rows, 69 KB, two workgroups per CU, so one's
+// memory phases overlap the other's solve.
+//
+// The unit-lower solves of gdn/chunk.rs:16-76 (separate products, four
+// interleaved partial sums, (s0+s2)+(s1+s3), scalar tail, one subtraction):
+// threads 0..127 the columns of U (rhs beta v), 128..255 those of W (rhs
+// (beta k) exp(g)), one column per thread, held in registers.  A lies in LDS
+// (in q's place, once dq is out) and is read as broadcast 16-byte words.
+// They are 4032 VALU instructions per wave, 13.4 us of a 2048-token layer's
+// four waves per (chunk, head).  As a launch of their own they also wrote and
+// read A and W's right-hand side: prep 31 + solve 38 us there.
 __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                             const float* __restrict__ v,
                                                              const float* __restrict__ beta,
                                                              const float* __restrict__ logd, int T, int H,
                                                              float* __restrict__ scratch) {
@@ -186,6 +195,7 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const float* __rest
         eg[tid] = cr_expf(gs[tid]);
         el[tid] = cr_expf(last - gs[tid]);
     }
+    f4m at[3];  // this wave's tiles of A, for LDS
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
         const int n = wv + 4 * m;
@@ -200,19 +210,30 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const float* __rest
         for (int r = 0; r < 4; ++r) {
             const int t = i0 + 4 * (lane >> 4) + r, s2 = j0 + (lane & 15);
             const float decay = s2 <= t ? cr_expf(gs[t] - gs[s2]) : 0.0f;
-            rec[kOffA + t * kC + s2] = a4[r] * decay;
+            at[m][r] = a4[r] * decay;
             rec[kOffIntra + t * kC + s2] = q4[r] * decay;
         }
     }
     __syncthreads();
-    // dq = q exp(g), dk = k exp(g_last - g), and the W right-hand side
-    // (beta k) exp(g)
+    // the right-hand sides: beta v, (beta k) exp(g)
+    const int col = tid & (kD - 1);
+    float xr[kC];
+    if (tid < kD) {
+#pragma unroll
+        for (int t = 0; t < kC; ++t) {
+            const float vv = t < rows ? v[((size_t)(t0 + t) * H + h) * kD + col] : 0.0f;
+            xr[t] = vv * bs[t];
+        }
+    } else {
+#pragma unroll
+        for (int t = 0; t < kC; ++t) xr[t] = (ks[t * kPad + col] * bs[t]) * eg[t];
+    }
+    // dq = q exp(g), dk = k exp(g_last - g)
 #pragma unroll
     for (int i = 0; i < kC * kD / 4 / 256; ++i) {
         const int f = tid + 256 * i, t = f >> 5, d = 4 * (f & 31);
-        const v4f qv = *(const v4f*)&qs[t * kPad + d], kv = *(const v4f*)&ks[t * kPad + d];
+        const v4f qv = *(const v4f*)&qs[t * kPad + d];
         *(v4f*)(rec + kOffDq + t * kD + d) = qv * eg[t];
-        *(v4f*)(rec + kOffW + t * kD + d) = (kv * bs[t]) * eg[t];
     }
     // dk in the scan's order: word (key d, four steps from t = 16 s4 + kq)
 #pragma unroll
@@ -227,47 +248,17 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const float* __rest
         *(v4f*)(rec + kOffDk + d * kC + 16 * kq + 4 * s4) = o;
     }
     if (tid < 64) rec[kOffDecay + tid] = cr_expf(gs[kC - 1]);  // replicated for vector loads
-}
-
-// Grid (chunks, H, 2), 128 threads: the unit-lower solves of gdn/chunk.rs:16-76
-// (separate products, four interleaved partial sums, (s0+s2)+(s1+s3), scalar
-// tail, one subtraction) for the 128 columns of U (z = 0, rhs beta v) or of
-// W (z = 1, rhs in place), one column per thread, held in registers.  The
-// coefficients are uniform across the wave and are read as scalar loads
-// through `amat` (the same records, never written here).
-__global__ __launch_bounds__(128) void gdn_chunk_solve_kernel(const float* __restrict__ v,
-                                                              const float* __restrict__ beta,
-                                                              const float* __restrict__ amat, int T, int H,
-                                                              float* __restrict__ scratch) {
-    // A is staged in LDS and read there as broadcast 16-byte reads: read
-    // from memory as scalar loads its 2016 coefficients outgrew the scalar
-    // registers, and the compiler parked them in vector-register lanes
-    // (a write and a read instruction per coefficient)
-    __shared__ float As[kC * kC];
-    const int c = blockIdx.x, h = blockIdx.y, z = blockIdx.z;
-    const int col = threadIdx.x;
-    const int t0 = c * kC, rows = min(kC, T - t0);
-    float* rec = scratch + ((size_t)c * H + h) * kRec;
-    const float* A = amat + ((size_t)c * H + h) * kRec + kOffA;
+    lds_barrier();  // q has been read
+    float* As = qs;
 #pragma unroll
-    for (int i = 0; i < kC * kC / (4 * 128); ++i)
-        *(v4f*)(As + 4 * (col + 128 * i)) = *(const v4f*)(A + 4 * (col + 128 * i));
-    __syncthreads();
-    float xr[kC];
-    if (z == 0) {
+    for (int m = 0; m < 3; ++m) {
+        const int n = wv + 4 * m;
+        if (n >= 10) break;
+        const int ti = n < 1 ? 0 : n < 3 ? 1 : n < 6 ? 2 : 3, tj = n - ti * (ti + 1) / 2;
 #pragma unroll
-        for (int t = 0; t < kC; ++t) {
-            float r = 0.0f;
-            if (t < rows) {
-                const float vv = v[((size_t)(t0 + t) * H + h) * kD + col];
-                r = vv * beta[(size_t)(t0 + t) * H + h];
-            }
-            xr[t] = r;
-        }
-    } else {
-#pragma unroll
-        for (int t = 0; t < kC; ++t) xr[t] = rec[kOffW + t * kD + col];
+        for (int r = 0; r < 4; ++r) As[(16 * ti + 4 * (lane >> 4) + r) * kC + 16 * tj + (lane & 15)] = at[m][r];
     }
+    lds_barrier();
 #pragma unroll
     for (int row = 0; row < kC; ++row) {
         const int vend = row / 4 * 4;
@@ -294,10 +285,7 @@ __global__ __launch_bounds__(128) void gdn_chunk_solve_kernel(const float* __res
         // hoisted further, the reads held most of A in registers
         if (row >= 1) asm volatile("" ::"v"(xr[row - 1]) : "memory");
     }
-    // W replaces its right-hand side in another column order: every column
-    // has been read
-    if (z != 0) __syncthreads();
-    float* dst = rec + (z == 0 ? kOffU + col : kOffW + perm_w(col));
+    float* dst = rec + (tid < kD ? kOffU + col : kOffW + perm_w(col));
 #pragma unroll
     for (int t = 0; t < kC; ++t) dst[t * kD] = xr[t];
 }
@@ -668,10 +656,8 @@ hipError_t gdn_chunk_prefill(const float* q, const float* k, const float* v, con
                              bool round_bf16, hipStream_t s) {
     if (T == 0 || H == 0 || (T + kC) * H * kD * 4 >= ((size_t)1 << 32)) return hipErrorInvalidValue;
     const unsigned nch = (unsigned)((T + kC - 1) / kC);
-    hipLaunchKernelGGL(gdn_chunk_prep_kernel, dim3(nch, (unsigned)H), dim3(256), 0, s, q, k, beta, logd, (int)T,
+    hipLaunchKernelGGL(gdn_chunk_prep_kernel, dim3(nch, (unsigned)H), dim3(256), 0, s, q, k, v, beta, logd, (int)T,
                        (int)H, scratch);
-    hipLaunchKernelGGL(gdn_chunk_solve_kernel, dim3(nch, (unsigned)H, 2), dim3(128), 0, s, v, beta,
-                       (const float*)scratch, (int)T, (int)H, scratch);
     hipLaunchKernelGGL(gdn_chunk_scan_kernel, dim3((unsigned)H, kD / kSW), dim3(512), 0, s, scratch, (int)T, (int)H,
                        state, key_major ? 1 : 0);
     const unsigned items = nch * (unsigned)H;
