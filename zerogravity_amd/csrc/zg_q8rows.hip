@@ -402,7 +402,9 @@ hipError_t launch_mfma_rows(const FusedGemvArgs& a, const int8_t* aq, const floa
     const size_t tiles = ((size_t)a.N + 15) / 16;
     // R 16-row tiles per wave task while the waves stay plentiful
     const int R = tiles >= 2 * 4096 ? 2 : 1;
-    const unsigned wgs = (unsigned)std::min<size_t>(((tiles + R - 1) / R + 3) / 4, 1024);
+    // two workgroups per CU are all that its registers hold: more only stage
+    // the activations again (151936 x 2048, 11 rows: 512 workgroups 105 us, 1024 116)
+    const unsigned wgs = (unsigned)std::min<size_t>(((tiles + R - 1) / R + 3) / 4, 512);
     // Activation rows per workgroup: at most 16 within 64 KB of LDS (two
     // workgroups per CU), the rows dealt evenly over as few workgroup rows as
     // that allows -- more when the tiles alone would leave CUs idle (each
