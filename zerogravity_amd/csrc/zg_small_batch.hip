@@ -15,11 +15,11 @@
 // and rows 8-15 those of unit p + 2; of the 16 x 16 product the two
 // diagonal 8 x 8 blocks are used, and added where the waves' sums are.
 //
-// Traced in a 3-row step (mfma16_q4k_kernel -> here, us): gate/up 8.6 -> 8.4,
-// down 8.3 -> 6.7, input 7.0 -> 6.6, output 5.6 -> 5.0, LM head 48.8 -> 40.9;
-// the step of 8 layers 367 -> 331.  What is left above the one-row GEMV (6.1,
-// 4.0, 5.1, 3.4, 31) is the dequantisation, 80 VALU instructions per wave
-// and 2048 weights.
+// Traced in a 3-row step (mfma16_q4k_kernel -> here, us): gate/up 8.6 -> 7.4,
+// down 8.3 -> 5.6, input 7.0 -> 6.6, output 5.6 -> 4.7, LM head 48.8 -> 39.1;
+// the step of 8 layers 368 -> 304.  A third of that is the finish: with four
+// rows per lane of half a wave, as the product lies in the registers, the
+// same kernels took 8.4, 6.7, 6.6, 5.0 and 40.9.
 #include <algorithm>
 
 #include "zg_decode_common.hpp"
@@ -91,14 +91,16 @@ __global__ __launch_bounds__(64 * W) void small_batch_q4k_kernel(FusedGemvArgs a
             }
     }
     load_tile(blockIdx.x);
-    // outputs of the finishing lanes: column o of the tile, rows 4 L + r
-    const int ncol = R == 16 ? n16 : n16 & 7;
-    const bool fin = L < 2 && (R == 16 || n16 < 8);
-    float yv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, gn = 0.0f;
-    if (EPI == EPI_RESID && w == 0 && fin) {
-        const int o = min((int)blockIdx.x * R + ncol, nout - 1);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) yv[r] = a.y[(size_t)min(4 * L + r, a.M - 1) * a.ldy + o];
+    // finishing lanes: one output each, row fm, column fn of the tile (16-row
+    // tiles without the GLU pairing: waves 0 and 1, eight columns each), so
+    // that the sums over the waves, the SiLU and the stores are not four
+    // in a row on a quarter of the lanes
+    constexpr int FW = R == 16 && EPI != EPI_GLU ? 2 : 1;
+    const int fr = lane & 3, fL = lane >> 5, fm = 4 * fL + fr, fn = ((lane >> 2) & 7) + 8 * w;
+    float yv = 0.0f, gn = 0.0f;
+    if (EPI == EPI_RESID && w < FW) {
+        const int o = min((int)blockIdx.x * R + fn, nout - 1);
+        yv = a.y[(size_t)min(fm, a.M - 1) * a.ldy + o];
         if (a.rms_tiles_out) gn = a.rms_gamma[o];
     }
     __builtin_amdgcn_sched_barrier(0);  // every load above is in flight before the first product
@@ -158,59 +160,56 @@ __global__ __launch_bounds__(64 * W) void small_batch_q4k_kernel(FusedGemvArgs a
         if (next < ntiles) load_tile(next);
         red[pb][w][lane] = acc;
         lds_barrier();
-        if (w == 0 && fin) {
-            // R = 8: the other diagonal block (lane n + 8, rows 8 on) joins
-            v4f v = red[pb][0][lane];
-            if (R == 8) v = v + red[pb][0][lane + 40];
+        if (w < FW) {
+            // element (column c, row fm) of wave q's product; R = 8: the other
+            // diagonal block (column c + 8, rows 8 on) joins
+            const float* base = (const float*)red[pb];
+            auto sum = [&](int c) {
+                float v = 0.0f;
 #pragma unroll
-            for (int q = 1; q < W; ++q) {
-                v = v + red[pb][q][lane];
-                if (R == 8) v = v + red[pb][q][lane + 40];
-            }
-            float vv[4] = {v.x, v.y, v.z, v.w};
-            if (a.rms_ss_in) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) vv[r] *= inv_s[4 * L + r];
-            }
-            const int o = t * TR + (EPI == EPI_GLU ? n16 & 7 : ncol);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = 4 * L + r;
-                if (EPI == EPI_GLU) {
-                    const float up = __shfl_xor(vv[r], 8, 16);  // the up row's sum
-                    if (n16 < 8 && o < nout) {
-                        // up * silu(gate), rounded to f16 into the down
-                        // projection's activation tiles (K2 = N/2 columns)
-                        const float pr = m < a.M ? up * ggml_silu(vv[r]) : 0.0f;
-                        if (a.status && !(fabsf(pr) <= 65504.0f)) atomicOr(a.status, 16);
-                        ((_Float16*)a.xh_out)[xh_tile_index(m, o, nout, a.M)] = (_Float16)pr;
-                    }
-                } else if (EPI == EPI_RESID) {
-                    const bool live = o < nout && m < a.M;
-                    const bool first = t == (int)blockIdx.x;
-                    float xn = 0.0f;
-                    if (live) {
-                        float* p = a.y + (size_t)m * a.ldy + o;
-                        xn = (first ? yv[r] : *p) + vv[r];  // source_binary Add, lib.rs:1258-1271
-                        *p = xn;
-                        if (!finite_f32(xn)) atomicOr(a.status, 1);
-                    }
-                    if (a.rms_tiles_out) {
-                        // the next RMS projection's A tile element and this
-                        // tile's sum of squares, as mfma16_q4k_kernel's
-                        const float g = first ? gn : (o < nout ? a.rms_gamma[o] : 0.0f);
-                        if (o < nout) {
-                            const float tv = live ? xn * g : 0.0f;
-                            if (!(fabsf(tv) <= 65504.0f)) atomicOr(a.status, 16);
-                            a.rms_tiles_out[xh_tile_index(m, o, N, a.M)] = (_Float16)tv;
-                        }
-                        const float sq = xn * xn;
-                        const double tot = R == 8 ? group8_sum_all((double)sq) : group_sum_last<16>((double)sq);
-                        if (n16 == R - 1) a.rms_ss_out[(size_t)m * (N / R) + t] = tot;
-                    }
-                } else if (o < nout && m < a.M) {
-                    a.y[(size_t)m * a.ldy + o] = vv[r];
+                for (int q = 0; q < W; ++q) {
+                    v += base[(q * 64 + c + 16 * fL) * 4 + fr];
+                    if (R == 8) v += base[(q * 64 + c + 8 + 16 * (fL + 2)) * 4 + fr];
                 }
+                return a.rms_ss_in ? v * inv_s[fm] : v;
+            };
+            const float v = sum(fn);
+            const int o = t * TR + fn;
+            const bool live = o < nout && fm < a.M;
+            if (EPI == EPI_GLU) {
+                // up * silu(gate), rounded to f16 into the down projection's
+                // activation tiles (K2 = N/2 columns)
+                const float pr = fm < a.M ? sum(fn + 8) * ggml_silu(v) : 0.0f;
+                if (live) {
+                    if (a.status && !(fabsf(pr) <= 65504.0f)) atomicOr(a.status, 16);
+                    ((_Float16*)a.xh_out)[xh_tile_index(fm, o, nout, a.M)] = (_Float16)pr;
+                }
+            } else if (EPI == EPI_RESID) {
+                const bool first = t == (int)blockIdx.x;
+                float xn = 0.0f;
+                if (live) {
+                    float* p = a.y + (size_t)fm * a.ldy + o;
+                    xn = (first ? yv : *p) + v;  // source_binary Add, lib.rs:1258-1271
+                    *p = xn;
+                    if (!finite_f32(xn)) atomicOr(a.status, 1);
+                }
+                if (a.rms_tiles_out) {
+                    // the next RMS projection's A tile element, as
+                    // mfma16_q4k_kernel's, and the sum of squares of the
+                    // eight columns
+                    if (live) {
+                        const float tv = xn * (first ? gn : a.rms_gamma[o]);
+                        if (!(fabsf(tv) <= 65504.0f)) atomicOr(a.status, 16);
+                        a.rms_tiles_out[xh_tile_index(fm, o, N, a.M)] = (_Float16)tv;
+                    }
+                    const float sq = xn * xn;
+                    double tot = (double)sq;
+#pragma unroll
+                    for (int off = 4; off < 32; off <<= 1) tot += __shfl_xor(tot, off, 64);
+                    if (live && (o & 7) == 0) a.rms_ss_out[(size_t)fm * (N >> 3) + (o >> 3)] = tot;
+                }
+            } else if (live) {
+                a.y[(size_t)fm * a.ldy + o] = v;
             }
         }
         pb ^= 1;
@@ -225,7 +224,7 @@ bool small_batch_fits(size_t M, size_t K, size_t N, int epi) {
 }
 
 int rms_ss_columns(size_t M, size_t K, size_t N) {
-    if (small_batch_fits(M, K, N, EPI_RESID)) return tile_rows(N, EPI_RESID);
+    if (small_batch_fits(M, K, N, EPI_RESID)) return 8;
     return batched16_supported(M, K, N, EPI_RESID) ? 16 : 32;
 }
 
