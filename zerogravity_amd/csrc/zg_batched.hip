@@ -345,7 +345,6 @@ __global__ __launch_bounds__(64 * kM16Waves) __attribute__((amdgpu_waves_per_eu(
     // block headers: one per block when a wave's units pair into blocks
     // (UPW even: units 2b, 2b+1 of block b), else one per unit
     constexpr int NH = UPW % 2 == 0 ? UPW / 2 : UPW;
-    static_assert(MBW * TMAX <= KW, "a finishing wave per (tile, row half)");
     __shared__ v4f red[KW][MBW * TMAX][64];
     __shared__ float inv_s[16 * MBW];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, L = lane >> 4, r16 = lane & 15;
@@ -420,19 +419,27 @@ __global__ __launch_bounds__(64 * kM16Waves) __attribute__((amdgpu_waves_per_eu(
             }
         }
     };
-    // a residual projection's own outputs, requested up front: wave w adds
-    // into (tile t0 + w/MBW, row half w%MBW) -- the single-pass shapes
-    float yv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, gn = 0.0f;
-    const bool ypre = EPI == EPI_RESID && LOOP == 0 && w < MBW * min(TMAX, t1 - t0);
-    if (ypre) {
-        const int n = (t0 + w / MBW) * 16 + r16;
-        if (n < N) {
+    // Finishing: element e of a pass is row 4 L + r of half mb, column n of
+    // tile t, e = (((t MBW + mb) 4 + L) CN + n) 4 + r, one per thread and
+    // round of 512, so that the sums over the waves, the SiLU or residual add
+    // and the stores run on every lane once or twice, not four rows in a row
+    // on the lanes and waves that hold them.
+    constexpr int CN = EPI == EPI_GLU ? 8 : 16, NE = 16 * CN;  // columns, elements per (tile, half)
+    constexpr int EPT = (TMAX * MBW * NE + 64 * KW - 1) / (64 * KW);
+    // a residual projection's own outputs, requested up front: the
+    // single-pass shapes
+    float yv[EPT], gn[EPT];
+    constexpr bool kPre = EPI == EPI_RESID && LOOP == 0;
+    if constexpr (kPre) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = m0 + 16 * (w % MBW) + 4 * L + r;
-                if (m < a.M) yv[r] = a.y[(size_t)m * a.ldy + n];
+        for (int i = 0; i < EPT; ++i) {
+            const int e = tid + 64 * KW * i, te = e / (NE * MBW);
+            const int n = (t0 + te) * 16 + ((e >> 2) & 15), m = m0 + 16 * ((e / NE) % MBW) + 4 * ((e >> 6) & 3) + (e & 3);
+            yv[i] = gn[i] = 0.0f;
+            if (t0 + te < t1 && te < TMAX && n < N) {
+                if (m < a.M) yv[i] = a.y[(size_t)m * a.ldy + n];
+                if (a.rms_tiles_out) gn[i] = a.rms_gamma[n];
             }
-            if (a.rms_tiles_out) gn = a.rms_gamma[n];
         }
     }
     v4u wA[UPW][TMAX], hA[NH][TMAX];
@@ -496,68 +503,59 @@ __global__ __launch_bounds__(64 * kM16Waves) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
             for (int mb = 0; mb < MBW; ++mb) red[w][MBW * t + mb][lane] = acc[t][mb];
         __syncthreads();
-        // wave w finishes (tile t = w/MBW, row half w%MBW)
-        if (w < MBW * ntb) {
-            v4f v = red[0][w][lane];
 #pragma unroll
-            for (int q = 1; q < KW; ++q) v = v + red[q][w][lane];
-            const int vt = tb + w / MBW, mh = 16 * (w % MBW);
-            float vv[4] = {v.x, v.y, v.z, v.w};
+        for (int i = 0; i < EPT; ++i) {
+            const int e = tid + 64 * KW * i, th = e / NE;  // th = t MBW + mb, uniform over a wave
+            if (th >= MBW * ntb) break;
+            const int r = e & 3, c = (e >> 2) & (CN - 1), ml = 4 * ((e / (4 * CN)) & 3) + r;
+            const int vt = tb + th / MBW, mh = 16 * (th % MBW) + ml, m = m0 + mh;
+            auto sum = [&](int col) {  // the waves' products of column col, in wave order
+                const float* base = (const float*)&red[0][th][col + 16 * (ml >> 2)] + r;
+                float v = base[0];
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (a.rms_ss_in) vv[r] *= inv_s[mh + 4 * L + r];
+                for (int q = 1; q < KW; ++q) v = v + base[q * MBW * TMAX * 64 * 4];
+                return a.rms_ss_in ? v * inv_s[mh] : v;
+            };
+            const float v = sum(c);
             if (EPI == EPI_GLU) {
-                const int j = vt * 8 + (r16 & 7);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float up = __shfl_xor(vv[r], 8, 16);  // the up row's sum (lane l ^ 8)
-                    const int m = m0 + mh + 4 * L + r;
-                    if (r16 < 8 && j < nout) {
-                        // up * silu(gate), rounded to f16 into the down
-                        // projection's activation tiles (K2 = N/2 columns)
-                        const float pr = m < a.M ? up * ggml_silu(vv[r]) : 0.0f;
-                        if (a.status && !(fabsf(pr) <= 65504.0f)) atomicOr(a.status, 16);
-                        ((_Float16*)a.xh_out)[xh_tile_index(m, j, nout, a.M)] = (_Float16)pr;
-                    }
+                const int j = vt * 8 + c;
+                if (j < nout) {
+                    // up * silu(gate), rounded to f16 into the down
+                    // projection's activation tiles (K2 = N/2 columns)
+                    const float pr = m < a.M ? sum(c + 8) * ggml_silu(v) : 0.0f;
+                    if (a.status && !(fabsf(pr) <= 65504.0f)) atomicOr(a.status, 16);
+                    ((_Float16*)a.xh_out)[xh_tile_index(m, j, nout, a.M)] = (_Float16)pr;
                 }
             } else if (EPI == EPI_RESID) {
-                const int n = vt * 16 + r16;
-                const bool nv = n < N;
-                float g = gn;
-                if (!ypre && nv && a.rms_tiles_out) g = a.rms_gamma[n];
+                const int n = vt * 16 + c;
+                const bool nv = n < N, live = nv && m < a.M;
+                float xn = 0.0f;
+                if (live) {
+                    float* p = a.y + (size_t)m * a.ldy + n;
+                    xn = (kPre ? yv[i] : *p) + v;  // source_binary Add, lib.rs:1258-1271
+                    *p = xn;
+                    if (!finite_f32(xn)) atomicOr(a.status, 1);
+                }
+                if (a.rms_tiles_out) {
+                    // the next RMS projection's A tile element (m, n):
+                    // f16(x_new * gamma) (its 1/rms is applied after its
+                    // dot), and this 16-column tile's f64 sum of the f32
+                    // squares of x_new (lanes 4 apart hold a row's columns)
+                    if (nv) {
+                        const float g = kPre ? gn[i] : a.rms_gamma[n];
+                        const float tv = live ? xn * g : 0.0f;
+                        if (!(fabsf(tv) <= 65504.0f)) atomicOr(a.status, 16);
+                        a.rms_tiles_out[xh_tile_index(m, n, N, a.M)] = (_Float16)tv;
+                    }
+                    const float sq = xn * xn;
+                    double tot = (double)sq;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int m = m0 + mh + 4 * L + r;
-                    const bool live = nv && m < a.M;
-                    float xn = 0.0f;
-                    if (live) {
-                        float* p = a.y + (size_t)m * a.ldy + n;
-                        xn = (ypre ? yv[r] : *p) + vv[r];  // source_binary Add, lib.rs:1258-1271
-                        *p = xn;
-                        if (!finite_f32(xn)) atomicOr(a.status, 1);
-                    }
-                    if (a.rms_tiles_out) {
-                        // the next RMS projection's A tile element (m, n):
-                        // f16(x_new * gamma) (its 1/rms is applied after its
-                        // dot), and this 16-column tile's f64 sum of the f32
-                        // squares of x_new (the 16 lanes of a row)
-                        if (nv) {
-                            const float tv = live ? xn * g : 0.0f;
-                            if (!(fabsf(tv) <= 65504.0f)) atomicOr(a.status, 16);
-                            a.rms_tiles_out[xh_tile_index(m, n, N, a.M)] = (_Float16)tv;
-                        }
-                        const float sq = xn * xn;
-                        const double tot = group_sum_last<16>((double)sq);
-                        if (r16 == 15) a.rms_ss_out[(size_t)m * (N >> 4) + vt] = tot;
-                    }
+                    for (int off = 4; off < 64; off <<= 1) tot += __shfl_xor(tot, off, 64);
+                    if (c == 0) a.rms_ss_out[(size_t)m * (N >> 4) + vt] = tot;
                 }
             } else {
-                const int n = vt * 16 + r16;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int m = m0 + mh + 4 * L + r;
-                    if (n < N && m < a.M) a.y[(size_t)m * a.ldy + n] = vv[r];
-                }
+                const int n = vt * 16 + c;
+                if (n < N && m < a.M) a.y[(size_t)m * a.ldy + n] = v;
             }
         }
         __syncthreads();
