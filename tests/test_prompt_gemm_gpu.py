@@ -53,3 +53,59 @@ def test_prompt_gemm_matches_float64(kern, M, N, K, norm):
     assert err.abs().max().item() <= 6e-3 * rms
     assert bool((y[M] == 7.0).all())  # nothing past the last row
     kern.release_source(700)
+
+
+def test_prompt_call_lays_out_the_allocation_free_rows(kern):
+    """A shape whose small batches read the 32-row tiles: the allocation-free
+    call finds them after a prompt alone."""
+    N, K = 300, 3584
+    rng = np.random.default_rng(9)
+    h = kern.register(701, "prompt.noalloc", synth.Q4_K, K, N, synth.random_q4_k(rng, N, K).reshape(-1))
+    x = torch.from_numpy(rng.standard_normal((256, K)).astype(np.float32)).cuda()
+    y = torch.empty(256, N, device="cuda")
+    y3, want = torch.empty(3, N, device="cuda"), torch.empty(3, N, device="cuda")
+    torch.cuda.synchronize()
+    kern.ctx.check(L.lib().zg_gemv_device(kern.ctx.h, h.h, x.data_ptr(), L.F32, 256, None, 1e-6, y.data_ptr(), None))
+    kern.ctx.check(L.lib().zg_gemv_device_noalloc(kern.ctx.h, h.h, x.data_ptr(), L.F32, 3, None, 1e-6, y3.data_ptr(),
+                                                  None))
+    kern.ctx.check(L.lib().zg_gemv_device(kern.ctx.h, h.h, x.data_ptr(), L.F32, 3, None, 1e-6, want.data_ptr(), None))
+    torch.cuda.synchronize()
+    assert torch.equal(y3, want)
+    kern.release_source(701)
+
+
+def test_captured_prompt_call_runs_unsplit_where_its_sums_do_not_fit():
+    """A longer prompt's activation leaves room for 300 rows, but not for
+    their four runs over K as well: the captured call does without them."""
+    from zerogravity_amd import regions as R
+    k = R.HipMatVecKernel(0)
+    N, K, M = 2048, 6144, 300
+    rng = np.random.default_rng(10)
+    h = k.register(702, "prompt.capture", synth.Q4_K, K, N, synth.random_q4_k(rng, N, K).reshape(-1))
+    x = torch.from_numpy(rng.standard_normal((1025, K)).astype(np.float32)).cuda()
+    big, y, want = (torch.zeros(m, N, device="cuda") for m in (1025, M, M))
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+
+    def call(m, out):
+        k.ctx.check(L.lib().zg_gemv_device(k.ctx.h, h.h, x.data_ptr(), L.F32, m, None, 1e-6, out.data_ptr(),
+                                           stream.cuda_stream))
+
+    call(1025, big)
+    stream.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+        call(M, y)
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        # the same products as the longer prompt's unsplit rows, in the same order up to the tile shape
+        diff = (y.double() - big[:M].double()).square().mean().sqrt()
+        assert diff <= 1e-5 * big[:M].double().square().mean().sqrt()
+    del graph
+    call(M, want)  # outside a capture: the buffer grows, K split
+    stream.synchronize()
+    assert (want.double() - y.double()).square().mean().sqrt() <= 1e-5 * y.double().square().mean().sqrt()
+    k.ctx.close()

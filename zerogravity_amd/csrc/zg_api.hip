@@ -527,18 +527,27 @@ int zg_gemv_device(zg_ctx* ctx, const zg_weight* w, const void* x, int x_dtype, 
             // Q4_K: a prompt's f16 weight tiles, or the 32-row tiles unless the
             // 16-row kernel takes this shape
             const bool prompt = w->dw.type == zg::kQ4_K && m_rows >= (size_t)zg::kGemmRows;
-            if (prompt && !w->dw.wh) {
+            // (a prompt lays out both, so that the allocation-free call finds
+            // the tiles its rows need)
+            const bool tiles = w->dw.type == zg::kQ4_K && !w->dw.qs_t &&
+                               !zg::batched16_supported(prompt ? 2 : m_rows, w->dw.K, w->dw.N, zg::EPI_STORE);
+            if (tiles || (prompt && !w->dw.wh)) {
                 ZG_HIP(hipStreamSynchronize(s));
-                ZG_HIP(zg::ensure_f16_tiles(const_cast<zg_weight*>(w)->dw, s));
-            } else if (!prompt && w->dw.type == zg::kQ4_K && !w->dw.qs_t &&
-                       !zg::batched16_supported(m_rows, w->dw.K, w->dw.N, zg::EPI_STORE)) {
-                ZG_HIP(hipStreamSynchronize(s));
-                ZG_HIP(zg::ensure_mfma_tiles(const_cast<zg_weight*>(w)->dw, s));
+                if (tiles) ZG_HIP(zg::ensure_mfma_tiles(const_cast<zg_weight*>(w)->dw, s));
+                if (prompt) ZG_HIP(zg::ensure_f16_tiles(const_cast<zg_weight*>(w)->dw, s));
             }
             // a prompt's partial sums behind its activation tiles
             const size_t act = align256(zg::batched_scratch_bytes(m_rows, w->dw.K));
             const int splits = prompt ? zg::prompt_splits(m_rows, w->dw.K, w->dw.N) : 1;
             f.prompt_parts_n = splits > 1 ? (size_t)splits * m_rows * w->dw.N : 0;
+            // a captured call cannot grow the buffer: it runs unsplit where
+            // only its activation fits
+            if (f.prompt_parts_n && ctx->actbuf.bytes >= act &&
+                ctx->actbuf.bytes < act + f.prompt_parts_n * sizeof(float)) {
+                hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+                ZG_HIP(hipStreamIsCapturing(s, &cs));
+                if (cs != hipStreamCaptureStatusNone) f.prompt_parts_n = 0;
+            }
             const size_t need = act + f.prompt_parts_n * sizeof(float);
             if (ctx->actbuf.bytes < need) ZG_HIP(hipStreamSynchronize(s));
             int rc = ensure(ctx, ctx->actbuf, need);

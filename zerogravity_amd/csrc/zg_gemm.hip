@@ -406,8 +406,16 @@ hipError_t prompt_gemm(const DeviceWeight& w, const FusedGemvArgs& args, const _
         const hipError_t e = launch_gemm<EPI_STORE>(a, SHAPE_128x128, xh, wh, s);
         if (e != hipSuccess) return e;
         const dim3 g((unsigned)(((size_t)a.M * a.N / 4 + 255) / 256));
-#define ZG_SUM(SV)                                                                                                 if (a.epi == EPI_RESID) hipLaunchKernelGGL((split_sum_kernel<SV, true>), g, dim3(256), 0, s, a);               else hipLaunchKernelGGL((split_sum_kernel<SV, false>), g, dim3(256), 0, s, a);
-        if (S == 4) { ZG_SUM(4) } else if (S == 3) { ZG_SUM(3) } else { ZG_SUM(2) }
+#define ZG_SUM(SV)                                                                                               \
+    if (a.epi == EPI_RESID) hipLaunchKernelGGL((split_sum_kernel<SV, true>), g, dim3(256), 0, s, a);               \
+    else hipLaunchKernelGGL((split_sum_kernel<SV, false>), g, dim3(256), 0, s, a);
+        if (S == 4) {
+            ZG_SUM(4)
+        } else if (S == 3) {
+            ZG_SUM(3)
+        } else {
+            ZG_SUM(2)
+        }
 #undef ZG_SUM
         return hipGetLastError();
     }

@@ -101,7 +101,7 @@ struct zg_session {
     void* xh = nullptr;  // f16 activations of the batched (B > 1) projections
     float* parts = nullptr;  // split-K partial tiles of residual projections (B > 1)
     void* xh3 = nullptr;     // the stream's RMS input tiles a residual projection leaves (B > 1)
-    double* rss = nullptr;   // and their per-tile sums of squares [rows][hidden/16 or hidden/32]
+    double* rss = nullptr;   // and their per-tile sums of squares [rows][hidden / rms_ss_columns]
     void* xh2 = nullptr;     // the SwiGLU product in f16 tiles, down projection input (B > 1)
     size_t y0w = 0;
     std::vector<float*> ring, rec;  // per GDN layer: conv ring [B][3W][4], state [B][2][H][128][128]
