@@ -307,7 +307,7 @@ __global__ __launch_bounds__(256) void fused_q8_kernel(FusedGemvArgs a) {
 // same order, bit for bit, on four times the waves.
 // What bounds it: launch, prologue and one memory round trip.  Against
 // fused_q8_kernel, whose waves take a group each (us, one row, N x K):
-// 1024 x 3584 9.4 -> 5.4 (32 -> 128 workgroups), 2048 x 6144 13.9 -> 9.2,
+// 1024 x 3584 9.4 -> 5.4 (32 -> 128 workgroups), 2048 x 6144 13.9 -> 7.9,
 // 1024 x 2048 5.8 -> 3.8; four rows 22.2 -> 8.3, 33.4 -> 19.4, 13.3 -> 8.6.
 template <int MT, int J, int CW, int PRO, int EPI>
 __global__ __launch_bounds__(256) void fused_q8_relay_kernel(FusedGemvArgs a) {
