@@ -86,7 +86,13 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_f16_kernel(FusedGemvArgs
     const int bm = 8 * band + tb % bw, bn = tb / bw;
     const int N = a.N, kf = a.K >> 4, mtiles = (a.M + 31) >> 5, ntiles = (N + 31) >> 5;
     // stage s covers fragments kFrags s ..; this run's stages [s0, s0 + ns)
-    const int s0 = z * (kf / kFrags) / S, ns = (z + 1) * (kf / kFrags) / S - s0;
+    const int s0 = z * (kf / kFrags) / S;
+    int ns = (z + 1) * (kf / kFrags) / S - s0;
+    // Opaque: with SwiGLU, where S is 1, the compiler otherwise peels the loop
+    // below and keeps two copies of the sums (registers of the 256 x 256,
+    // 128 x 256 and 128 x 128 shapes: 256 and 254 spilled, 182, 104; with
+    // this 184, 102, 60).  8192 x 12288 x 2048: 2379 -> 385 us.
+    asm volatile("" : "+s"(ns));
 
     // Weight tile of slot b of this workgroup: wave wn's slots are 2 wn and
     // 2 wn + 1; with SwiGLU slot 2 wn is a gate tile and 2 wn + 1 the up tile
