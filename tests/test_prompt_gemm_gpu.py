@@ -74,38 +74,40 @@ def test_prompt_call_lays_out_the_allocation_free_rows(kern):
     kern.release_source(701)
 
 
-def test_captured_prompt_call_runs_unsplit_where_its_sums_do_not_fit():
-    """A longer prompt's activation leaves room for 300 rows, but not for
-    their four runs over K as well: the captured call does without them."""
+def test_captured_prompt_call_outlives_later_calls():
+    """A captured prompt whose K is split keeps its buffers through later
+    ordinary calls: of its own shape, of a shorter prompt (whose sums are
+    larger than its own), of one with other sums.  The graph is replayed
+    after all of them, bit for bit what the ordinary call gives."""
     from zerogravity_amd import regions as R
     k = R.HipMatVecKernel(0)
     N, K, M = 2048, 6144, 300
     rng = np.random.default_rng(10)
     h = k.register(702, "prompt.capture", synth.Q4_K, K, N, synth.random_q4_k(rng, N, K).reshape(-1))
     x = torch.from_numpy(rng.standard_normal((1025, K)).astype(np.float32)).cuda()
-    big, y, want = (torch.zeros(m, N, device="cuda") for m in (1025, M, M))
+    out = {m: torch.zeros(m, N, device="cuda") for m in (256, M, 601, 1025)}
+    y = torch.zeros(M, N, device="cuda")
     stream = torch.cuda.Stream()
     torch.cuda.synchronize()
 
-    def call(m, out):
-        k.ctx.check(L.lib().zg_gemv_device(k.ctx.h, h.h, x.data_ptr(), L.F32, m, None, 1e-6, out.data_ptr(),
+    def call(m, to):
+        k.ctx.check(L.lib().zg_gemv_device(k.ctx.h, h.h, x.data_ptr(), L.F32, m, None, 1e-6, to.data_ptr(),
                                            stream.cuda_stream))
 
-    call(1025, big)
+    call(1025, out[1025])
     stream.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
         call(M, y)
-    for _ in range(3):
+    for m in (M, 256, 601, 1025, M):
+        call(m, out[m])
+        stream.synchronize()
         y.zero_()
         torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
-        # the same products as the longer prompt's unsplit rows, in the same order up to the tile shape
-        diff = (y.double() - big[:M].double()).square().mean().sqrt()
-        assert diff <= 1e-5 * big[:M].double().square().mean().sqrt()
-    del graph
-    call(M, want)  # outside a capture: the buffer grows, K split
-    stream.synchronize()
-    assert (want.double() - y.double()).square().mean().sqrt() <= 1e-5 * y.double().square().mean().sqrt()
+        # the same products as the longer prompt's unsplit rows, in another order of summation
+        diff = (y.double() - out[1025][:M].double()).square().mean().sqrt()
+        assert diff <= 1e-5 * out[1025][:M].double().square().mean().sqrt()
+    assert torch.equal(y, out[M])
     k.ctx.close()

@@ -227,6 +227,7 @@ void zg_ctx_destroy(zg_ctx* ctx) {
         ctx->weights.clear();
         if (ctx->scratch.ptr) (void)hipFree(ctx->scratch.ptr);
         if (ctx->actbuf.ptr) (void)hipFree(ctx->actbuf.ptr);
+        if (ctx->sumbuf.ptr) (void)hipFree(ctx->sumbuf.ptr);
         if (ctx->chunkbuf.ptr) (void)hipFree(ctx->chunkbuf.ptr);
         if (ctx->d_flag) (void)hipFree(ctx->d_flag);
         (void)hipStreamDestroy(ctx->stream);
@@ -536,23 +537,28 @@ int zg_gemv_device(zg_ctx* ctx, const zg_weight* w, const void* x, int x_dtype, 
                 if (tiles) ZG_HIP(zg::ensure_mfma_tiles(const_cast<zg_weight*>(w)->dw, s));
                 if (prompt) ZG_HIP(zg::ensure_f16_tiles(const_cast<zg_weight*>(w)->dw, s));
             }
-            // a prompt's partial sums behind its activation tiles
-            const size_t act = align256(zg::batched_scratch_bytes(m_rows, w->dw.K));
-            const int splits = prompt ? zg::prompt_splits(m_rows, w->dw.K, w->dw.N) : 1;
-            f.prompt_parts_n = splits > 1 ? (size_t)splits * m_rows * w->dw.N : 0;
-            // a captured call cannot grow the buffer: it runs unsplit where
-            // only its activation fits
-            if (f.prompt_parts_n && ctx->actbuf.bytes >= act &&
-                ctx->actbuf.bytes < act + f.prompt_parts_n * sizeof(float)) {
-                hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-                ZG_HIP(hipStreamIsCapturing(s, &cs));
-                if (cs != hipStreamCaptureStatusNone) f.prompt_parts_n = 0;
-            }
-            const size_t need = act + f.prompt_parts_n * sizeof(float);
+            const size_t need = zg::batched_scratch_bytes(m_rows, w->dw.K);
             if (ctx->actbuf.bytes < need) ZG_HIP(hipStreamSynchronize(s));
             int rc = ensure(ctx, ctx->actbuf, need);
             if (rc) return rc;
-            if (f.prompt_parts_n) f.prompt_parts = (float*)((char*)ctx->actbuf.ptr + act);
+            if (prompt) {
+                // the runs over K sum in a buffer of their own, of the bound
+                // of every prompt and never moved, so that no later call
+                // frees what a captured one names.  The first prompt outside
+                // a capture makes it; a prompt without it runs unsplit.
+                hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+                if (!ctx->sumbuf.ptr) ZG_HIP(hipStreamIsCapturing(s, &cs));
+                if (!ctx->sumbuf.ptr && cs == hipStreamCaptureStatusNone) {
+                    if (hipMalloc(&ctx->sumbuf.ptr, zg::kPromptParts * sizeof(float)) == hipSuccess) {
+                        ctx->sumbuf.bytes = zg::kPromptParts * sizeof(float);
+                    } else {
+                        (void)hipGetLastError();
+                        ctx->sumbuf.ptr = nullptr;
+                    }
+                }
+                f.prompt_parts = (float*)ctx->sumbuf.ptr;
+                f.prompt_parts_n = ctx->sumbuf.bytes / sizeof(float);
+            }
             ZG_HIP(zg::batched_gemv(w->dw, f, ctx->actbuf.ptr, s));
         } else {
             ZG_HIP(zg::fused_gemv(w->dw, f, s));

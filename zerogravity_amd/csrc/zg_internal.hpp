@@ -313,6 +313,9 @@ uint64_t prompt_gemm_bytes(size_t M, size_t K, size_t N);
 // Runs over K the prompt GEMM takes when given a workspace (prompt_parts) of
 // that many M x N partial sums; 1: none.
 int prompt_splits(size_t M, size_t K, size_t N);
+// Floats that hold any prompt's partial sums: splits times tiles stay within
+// 256 workgroups of 128 x 128 outputs.
+constexpr size_t kPromptParts = 256 * 128 * 128;
 
 // GDN decode: conv (4-slot ring per channel) + SiLU + q/k L2 + gates +
 // recurrence for B rows.  proj rows: [qkv (3W) | z (W) | alpha (H) | beta (H)].

@@ -1285,9 +1285,6 @@ int prefill_batched_body(zg_session* s, size_t row, size_t n, const uint32_t* to
             return fail(ctx, ZG_E_LIMIT, "prompt too long for the batched prefill (an operand of its projections "
                                          "would reach 4 GiB): split it over several calls");
     enum { X, P, Q, K, V, BETA, LOGD, CORE, QB, OB, XH, XH2, CHUNK, TOK, ATTP, RPARTS, NBUF };
-    // the split residual projections' partial sums: splits times tiles stay
-    // within 256 workgroups of 128 x 128 outputs (prompt_splits)
-    const size_t kSplitParts = 256 * 128 * 128;
     if (n > s->pf_cap) {
         ZG_HIP(hipStreamSynchronize(st));
         for (void* p : s->pf) (void)hipFree(p);
@@ -1297,7 +1294,7 @@ int prefill_batched_body(zg_session* s, size_t row, size_t n, const uint32_t* to
                                     n * GH * 4, mpad * W * 4, n * QD * 4, mpad * QD * 4,
                                     zg::batched_scratch_bytes(n, std::max({H, F, W, QD})),
                                     zg::batched_scratch_bytes(n, F), zg::gdn_chunk_scratch_bytes(n, GH), n * 4,
-                                    zg::attn_prefill_part_bytes(n, (int)g.q_heads), kSplitParts * 4};
+                                    zg::attn_prefill_part_bytes(n, (int)g.q_heads), zg::kPromptParts * 4};
         for (int i = 0; i < NBUF; ++i) {
             ZG_HIP(hipMalloc(&s->pf[i], std::max<size_t>(bytes[i], 256)));
             ZG_HIP(hipMemsetAsync(s->pf[i], 0, std::max<size_t>(bytes[i], 256), st));  // stream-ordered
@@ -1332,7 +1329,7 @@ int prefill_batched_body(zg_session* s, size_t row, size_t n, const uint32_t* to
         f.xh_in = xh_in;
         if (epi == zg::EPI_RESID && ldy == H) {
             f.prompt_parts = (float*)s->pf[RPARTS];
-            f.prompt_parts_n = kSplitParts;
+            f.prompt_parts_n = zg::kPromptParts;
         }
         return zg::batched_gemv(w->dw, f, s->pf[XH], st);
     };
