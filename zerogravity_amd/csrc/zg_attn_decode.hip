@@ -618,12 +618,8 @@ int attn_split_span(size_t B, int nkv, size_t max_ctx) {
     const size_t target = B <= 4 ? 256 : 512;
     const size_t want = (max_ctx * B * (size_t)nkv + target - 1) / target;
     const size_t floor = (max_ctx + kSplitMaxChunks - 1) / kSplitMaxChunks;
-    const size_t s = (std::max({want, floor, (size_t)32}) + 31) / 32 * 32;
-    // beyond 4 rows the target is what the CUs hold at once: a 32-token step
-    // more rather than a few workgroups in a second round (24 rows of 1024
-    // tokens: 528 workgroups of 96 tokens 26.0 us, 384 of 128 21.0)
-    const bool over = B > 4 && (max_ctx + s - 1) / s * B * (size_t)nkv > target;
-    return (int)(over && s + 32 <= (size_t)kSplitMaxSpan ? s + 32 : s);
+    const size_t s = std::max({want, floor, (size_t)32});
+    return (int)((s + 31) / 32 * 32);
 }
 
 int attn_split_chunks(size_t B, int nkv, size_t max_ctx) {
