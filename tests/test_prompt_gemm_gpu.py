@@ -74,6 +74,31 @@ def test_prompt_call_lays_out_the_allocation_free_rows(kern):
     kern.release_source(701)
 
 
+def test_a_new_layout_is_written_before_another_stream_finds_it(kern):
+    """The first prompt of a large weight on one stream builds its 32-row
+    tiles; an allocation-free call on another stream reads them at once."""
+    N, K = 40000, 3584
+    rng = np.random.default_rng(12)
+    w = synth.random_q4_k(rng, 2000, K).reshape(-1)
+    h = kern.register(703, "prompt.streams", synth.Q4_K, K, N, np.tile(w, 20))
+    x = torch.from_numpy(rng.standard_normal((256, K)).astype(np.float32)).cuda()
+    y = torch.empty(256, N, device="cuda")
+    y3, want = torch.empty(3, N, device="cuda"), torch.empty(3, N, device="cuda")
+    one, two = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    kern.ctx.check(L.lib().zg_gemv_device(kern.ctx.h, h.h, x.data_ptr(), L.F32, 256, None, 1e-6, y.data_ptr(),
+                                          one.cuda_stream))
+    kern.ctx.check(L.lib().zg_gemv_device_noalloc(kern.ctx.h, h.h, x.data_ptr(), L.F32, 3, None, 1e-6, y3.data_ptr(),
+                                                  two.cuda_stream))
+    torch.cuda.synchronize()
+    kern.ctx.check(L.lib().zg_gemv_device_noalloc(kern.ctx.h, h.h, x.data_ptr(), L.F32, 3, None, 1e-6,
+                                                  want.data_ptr(), two.cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(y3, want)
+    assert torch.equal(y3[:, :2000], y3[:, 38000:])
+    kern.release_source(703)
+
+
 def test_captured_prompt_call_outlives_later_calls():
     """A captured prompt whose K is split keeps its buffers through later
     ordinary calls: of its own shape, of a shorter prompt (whose sums are

@@ -722,6 +722,8 @@ hipError_t ensure_mfma_tiles(DeviceWeight& w, hipStream_t s) {
     hipLaunchKernelGGL(mfma_tile_q4k_kernel, dim3((unsigned)tiles, (unsigned)nbk), dim3(256), 0, s,
                        (const uint8_t*)w.qs, (const v4u*)w.hdr, (int)w.N, (int)w.K, (v4u*)q, (v4u*)h);
     e = hipGetLastError();
+    // written before any stream can find it
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
         (void)hipFree(q);
         (void)hipFree(h);

@@ -363,6 +363,8 @@ hipError_t ensure_f16_tiles(DeviceWeight& w, hipStream_t s) {
     hipLaunchKernelGGL(f16_tile_q4k_kernel, dim3((unsigned)tiles, (unsigned)(w.K / 256)), dim3(256), 0, s,
                        (const uint8_t*)w.qs, (const v4u*)w.hdr, (int)w.N, (int)w.K, (_Float16*)p);
     e = hipGetLastError();
+    // written before any stream can find it
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
         (void)hipFree(p);
         return e;

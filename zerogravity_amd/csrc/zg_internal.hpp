@@ -282,8 +282,9 @@ hipError_t fused_gemv(const DeviceWeight& w, const FusedGemvArgs& a, hipStream_t
 // values rounded to f16 into `scratch` (batched_scratch_bytes), then an f16
 // MFMA GEMM with the epilogue (LDS-staged from 1024 rows).
 size_t batched_scratch_bytes(size_t M, size_t K);
-// Builds w.qs_t / w.hdr_t (Q4_K) if absent: allocates, so call it outside
-// graph capture.  batched_gemv refuses a Q4_K weight without them.
+// Builds w.qs_t / w.hdr_t (Q4_K) if absent: allocates and waits for the
+// stream, so call it outside graph capture.  batched_gemv refuses a Q4_K
+// weight without them.
 hipError_t ensure_mfma_tiles(DeviceWeight& w, hipStream_t s);
 // Builds w.wh (Q4_K) if absent, likewise: batched_gemv refuses a prompt
 // (M >= kGemmRows) without it.

@@ -924,7 +924,6 @@ int zg_session_create(zg_model* m, size_t max_batch, size_t max_context, int kv_
                 const hipError_t e = zg::ensure_mfma_tiles(w->dw, ctx->stream);
                 if (e != hipSuccess) return fail(ctx, ZG_E_RESOURCE, "MFMA tile layout of a Q4_K weight");
             }
-        if (hipStreamSynchronize(ctx->stream) != hipSuccess) return fail(ctx, ZG_E_DEVICE, "tile layout build");
     }
     auto s = new zg_session();
     s->m = m;
