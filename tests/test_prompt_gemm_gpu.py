@@ -74,6 +74,45 @@ def test_prompt_call_lays_out_the_allocation_free_rows(kern):
     kern.release_source(701)
 
 
+@pytest.mark.parametrize("K", [3584, 2048])
+@pytest.mark.parametrize("M", [256, 449, 600])
+def test_captured_prompt_call_of_a_weight_without_prompt_tiles(K, M):
+    """A weight that only smaller calls have used: the captured prompt runs on
+    the 32-row tiles those left, or on the weight's own layout where they
+    need none.  Its products are the prompt GEMM's, summed in another order."""
+    from zerogravity_amd import regions as R
+    k = R.HipMatVecKernel(0)
+    N = 1000
+    rng = np.random.default_rng(K + M)
+    h, other = (k.register(704, f"prompt.late.{i}", synth.Q4_K, K, N, synth.random_q4_k(rng, N, K).reshape(-1))
+                for i in range(2))
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).cuda()
+    y, want = torch.zeros(M + 1, N, device="cuda"), torch.zeros(M, N, device="cuda")
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+
+    def call(w, m, to):
+        k.ctx.check(L.lib().zg_gemv_device(k.ctx.h, w.h, x.data_ptr(), L.F32, m, None, 1e-6, to.data_ptr(),
+                                           stream.cuda_stream))
+
+    call(other, M, want)  # the activation buffer's size
+    call(h, 200, want)
+    stream.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+        call(h, M, y)
+    call(h, M, want)
+    for _ in range(3):
+        y.fill_(7.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        diff = (y[:M].double() - want.double()).square().mean().sqrt()
+        assert diff <= 1e-5 * want.double().square().mean().sqrt()
+        assert bool((y[M] == 7.0).all())
+    k.ctx.close()
+
+
 def test_a_new_layout_is_written_before_another_stream_finds_it(kern):
     """The first prompt of a large weight on one stream builds its 32-row
     tiles; an allocation-free call on another stream reads them at once."""

@@ -1,5 +1,6 @@
 // C ABI of the gfx950 backend (include/zg_hip.h): context, resident weight
 // cache, boundary-A region entry points and the device GEMV API.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <atomic>
@@ -532,7 +533,11 @@ int zg_gemv_device(zg_ctx* ctx, const zg_weight* w, const void* x, int x_dtype, 
             // the tiles its rows need)
             const bool tiles = w->dw.type == zg::kQ4_K && !w->dw.qs_t &&
                                !zg::batched16_supported(prompt ? 2 : m_rows, w->dw.K, w->dw.N, zg::EPI_STORE);
-            if (tiles || (prompt && !w->dw.wh)) {
+            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+            if (tiles || (prompt && (!w->dw.wh || !ctx->sumbuf.ptr))) ZG_HIP(hipStreamIsCapturing(s, &cs));
+            // a captured call takes the layouts that are there
+            const bool capturing = cs != hipStreamCaptureStatusNone;
+            if (!capturing && (tiles || (prompt && !w->dw.wh))) {
                 ZG_HIP(hipStreamSynchronize(s));
                 if (tiles) ZG_HIP(zg::ensure_mfma_tiles(const_cast<zg_weight*>(w)->dw, s));
                 if (prompt) ZG_HIP(zg::ensure_f16_tiles(const_cast<zg_weight*>(w)->dw, s));
@@ -546,9 +551,7 @@ int zg_gemv_device(zg_ctx* ctx, const zg_weight* w, const void* x, int x_dtype, 
                 // of every prompt and never moved, so that no later call
                 // frees what a captured one names.  The first prompt outside
                 // a capture makes it; a prompt without it runs unsplit.
-                hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-                if (!ctx->sumbuf.ptr) ZG_HIP(hipStreamIsCapturing(s, &cs));
-                if (!ctx->sumbuf.ptr && cs == hipStreamCaptureStatusNone) {
+                if (!ctx->sumbuf.ptr && !capturing) {
                     if (hipMalloc(&ctx->sumbuf.ptr, zg::kPromptParts * sizeof(float)) == hipSuccess) {
                         ctx->sumbuf.bytes = zg::kPromptParts * sizeof(float);
                     } else {
@@ -559,7 +562,17 @@ int zg_gemv_device(zg_ctx* ctx, const zg_weight* w, const void* x, int x_dtype, 
                 f.prompt_parts = (float*)ctx->sumbuf.ptr;
                 f.prompt_parts_n = ctx->sumbuf.bytes / sizeof(float);
             }
-            ZG_HIP(zg::batched_gemv(w->dw, f, ctx->actbuf.ptr, s));
+            // a prompt without a layout for one: rows by rows on the 16-row
+            // kernel, which reads the weight's own (batched_gemv refuses the
+            // shapes it does not take): M = 512, N = K = 2048 45 us against 21
+            const bool slices = prompt && !w->dw.wh && !w->dw.qs_t;
+            const size_t step = slices ? (size_t)zg::kGemmRows - 32 : m_rows;
+            for (size_t m = 0; m < m_rows; m += step) {
+                f.M = (int)std::min(step, m_rows - m);
+                f.x = (const float*)x + m * w->dw.K;
+                f.y = y + m * w->dw.N;
+                ZG_HIP(zg::batched_gemv(w->dw, f, ctx->actbuf.ptr, s));
+            }
         } else {
             ZG_HIP(zg::fused_gemv(w->dw, f, s));
         }

@@ -821,12 +821,15 @@ hipError_t batched_gemv(const DeviceWeight& w, const FusedGemvArgs& args, void* 
     if (w.type != kQ4_K || w.K % 256 || w.K > 8192 || args.M <= 0 || args.M > 65535 * 32) return hipErrorInvalidValue;
     if (args.pro == PRO_GATED && args.group != 128) return hipErrorInvalidValue;
     const bool m16 = batched16_supported((size_t)args.M, w.K, w.N, args.epi);
+    if (args.M >= kGemmRows && prompt_gemm_bytes((size_t)args.M, w.K, w.N) >= ((uint64_t)1 << 32))
+        return hipErrorInvalidValue;
     // prompt-sized M: the f16 GEMM (zg_gemm.hip); a pending split-K or RMS
-    // tiles belong to the decode step's 32-row kernel
-    const bool prompt = args.M >= kGemmRows && !(args.epi == EPI_RESID && args.splits > 1 && args.parts) &&
+    // tiles belong to the decode step's 32-row kernel, which also takes a
+    // prompt whose weight has no f16 tiles (a call captured before any
+    // prompt): M = 512, N = 2048, K = 3584 48 against 25 us
+    const bool prompt = args.M >= kGemmRows && w.wh && !(args.epi == EPI_RESID && args.splits > 1 && args.parts) &&
                         !args.rms_tiles_out && !args.rms_ss_in && prompt_gemm_supported(w.type, w.K, w.N, args.epi);
-    // ensure_f16_tiles / ensure_mfma_tiles first
-    if (prompt ? !w.wh : !m16 && (!w.qs_t || !w.hdr_t)) return hipErrorNotReady;
+    if (!prompt && !m16 && (!w.qs_t || !w.hdr_t)) return hipErrorNotReady;  // ensure_f16_tiles / ensure_mfma_tiles first
     FusedGemvArgs a = args;
     a.qs = m16 ? w.qs : w.qs_t;  // the 16-row kernel reads the Q4_K tile layout itself
     a.hdr = m16 ? w.hdr : w.hdr_t;

@@ -399,7 +399,6 @@ int prompt_splits(size_t M, size_t K, size_t N) {
 hipError_t prompt_gemm(const DeviceWeight& w, const FusedGemvArgs& args, const _Float16* xh, hipStream_t s) {
     if (!prompt_gemm_supported(w.type, w.K, w.N, args.epi) || !w.wh || args.M <= 0) return hipErrorInvalidValue;
     if (args.epi == EPI_GLU && !args.xh_out) return hipErrorInvalidValue;
-    if (prompt_gemm_bytes((size_t)args.M, w.K, w.N) >= ((uint64_t)1 << 32)) return hipErrorInvalidValue;
     FusedGemvArgs a = args;
     a.K = (int)w.K;
     a.N = (int)w.N;
