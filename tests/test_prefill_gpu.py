@@ -130,6 +130,27 @@ def test_prefill_batched_refusals(kern, tiny):
     m8.close()
 
 
+@pytest.mark.parametrize("n", [100, 300])
+def test_prefill_leaves_the_allocation_free_rows_their_layout(kern, tiny, n):
+    """After a prefill of any length the allocation-free call takes the
+    model's weights (K = 512: its rows read the 32-row tiles)."""
+    import torch
+    m = qwen35.QwenModelHip(TINY, tiny, kernel=kern)
+    s = m.session(max_batch=1, max_context=512, kv_dtype=L.F32)
+    s.prefill_batched(_tokens(3, n, TINY["vocab"]))
+    codec, k, rows, data = tiny["blk.0.ffn_down.weight"]
+    w = kern.register(m.source_id, "blk.0.ffn_down.weight", codec, k, rows, data)
+    x = torch.randn(3, k, device="cuda")
+    y, want = torch.zeros(3, rows, device="cuda"), torch.zeros(3, rows, device="cuda")
+    torch.cuda.synchronize()
+    for fn, to in ((L.lib().zg_gemv_device_noalloc, y), (L.lib().zg_gemv_device, want)):
+        kern.ctx.check(fn(kern.ctx.h, w.h, x.data_ptr(), L.F32, 3, None, 1e-6, to.data_ptr(), None))
+    torch.cuda.synchronize()
+    assert torch.equal(y, want)
+    m.close()
+    kern.release_source(m.source_id)
+
+
 @pytest.mark.parametrize("kv", [L.BF16, L.F32])
 def test_prefill_batched_2b_shapes(kern, kv):
     """The 2B layer shapes (16 GDN heads, 8 query / 2 KV heads, FFN 6144) over

@@ -1271,9 +1271,12 @@ int prefill_batched_body(zg_session* s, size_t row, size_t n, const uint32_t* to
     // them, and must find every other row as the host has it)
     int rc0 = sync_positions(s, st);
     if (rc0) return rc0;
-    for (zg_weight* w : ws)
+    // (the 32-row tiles at any length: the allocation-free call, which takes
+    // fewer rows, finds them after a prefill)
+    for (zg_weight* w : ws) {
+        if (!zg::xh16_layout(1, w->dw.K)) ZG_HIP(zg::ensure_mfma_tiles(w->dw, st));
         if (n >= (size_t)zg::kGemmRows) ZG_HIP(zg::ensure_f16_tiles(w->dw, st));
-        else if (!zg::xh16_layout(n, w->dw.K)) ZG_HIP(zg::ensure_mfma_tiles(w->dw, st));
+    }
     const size_t H = g.hidden, F = g.ffn, W = (size_t)g.gdn_heads * g.gdn_dim, GH = g.gdn_heads;
     const size_t QD = (size_t)g.q_heads * g.head_dim;
     const size_t mpad = (n + 31) / 32 * 32;
