@@ -231,6 +231,36 @@ def test_prefill_batched_prompt_gemm_matches_oracle(kern, n):
     m.close()
 
 
+def test_prefill_where_the_f16_tiles_do_not_fit(kern):
+    """With less memory free than the model's f16 tiles take, a long prompt's
+    projections run on the 32-row tiles; with room again, on the prompt GEMM:
+    the same products in another order before their roundings to f16."""
+    import torch
+    t = qwen35.synthetic_tensors(WIDE, gguf.Q4_K, seed=8)
+    m = qwen35.QwenModelHip(WIDE, t, kernel=kern)
+    s = m.session(max_batch=1, max_context=320, kv_dtype=L.F32)
+    toks = _tokens(11, 300, WIDE["vocab"])
+    room = 300 << 20  # the f16 tiles take 470 MB, the buffers and the 32-row tiles half of this
+    full = []
+    torch.cuda.empty_cache()
+    for _ in range(4):
+        left = torch.cuda.mem_get_info()[0] - room
+        if left > 1 << 24:
+            full.append(torch.empty(left, dtype=torch.uint8, device="cuda"))
+    try:
+        lg0, st0 = s.prefill_batched(toks), s.state()
+    finally:
+        del full
+        torch.cuda.empty_cache()
+    s.reset()
+    lg1, st1 = s.prefill_batched(toks), s.state()
+    worst = float(np.max(np.abs(lg0 - lg1)))
+    print(f"prefill on the 32-row tiles against the f16 tiles: logits max-abs {worst:.3e}")
+    assert 0 < worst <= LOGIT_TOL and int(np.argmax(lg0)) == int(np.argmax(lg1))
+    assert rel_err(st0, st1) <= 1e-2
+    m.close()
+
+
 def test_prefill_batched_8192_matches_oracle(kern):
     """The longest prompt the bench times: 8192 tokens at the 2B widths (4
     layers, bf16 KV) through zg_prefill_batched -- prompt GEMM, chunked GDN

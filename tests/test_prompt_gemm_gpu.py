@@ -113,6 +113,41 @@ def test_captured_prompt_call_of_a_weight_without_prompt_tiles(K, M):
     k.ctx.close()
 
 
+@pytest.mark.parametrize("K", [7168, 4096])
+def test_prompt_call_where_the_f16_tiles_do_not_fit(K):
+    """With less memory free than the f16 tiles take, a prompt runs on the
+    32-row tiles (K = 7168) or the weight's own layout (K = 4096)."""
+    from zerogravity_amd import regions as R
+    k = R.HipMatVecKernel(0)
+    N, M = 65536, 300
+    rng = np.random.default_rng(K)
+    h = k.register(705, "prompt.full", synth.Q4_K, K, N, np.tile(synth.random_q4_k(rng, 2048, K).reshape(-1), 32))
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).cuda()
+    y, want = torch.zeros(M, N, device="cuda"), torch.zeros(M, N, device="cuda")
+    torch.cuda.synchronize()
+
+    def call(to):
+        k.ctx.check(L.lib().zg_gemv_device(k.ctx.h, h.h, x.data_ptr(), L.F32, M, None, 1e-6, to.data_ptr(), None))
+        torch.cuda.synchronize()
+
+    torch.cuda.empty_cache()
+    room = N * K * 2 * 7 // 8  # the 32-row tiles and the buffers fit, the f16 tiles do not
+    full = []
+    for _ in range(4):  # (less is reported free than the first of them leaves)
+        left = torch.cuda.mem_get_info()[0] - room
+        if left > 1 << 24:
+            full.append(torch.empty(left, dtype=torch.uint8, device="cuda"))
+    try:
+        call(y)
+    finally:
+        del full
+        torch.cuda.empty_cache()
+    call(want)  # the prompt GEMM: the same products in another order
+    assert (y.double() - want.double()).square().mean().sqrt() <= 1e-5 * want.double().square().mean().sqrt()
+    assert not torch.equal(y, want)  # (they were other kernels)
+    k.ctx.close()
+
+
 def test_a_new_layout_is_written_before_another_stream_finds_it(kern):
     """The first prompt of a large weight on one stream builds its 32-row
     tiles; an allocation-free call on another stream reads them at once."""

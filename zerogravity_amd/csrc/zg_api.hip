@@ -540,7 +540,11 @@ int zg_gemv_device(zg_ctx* ctx, const zg_weight* w, const void* x, int x_dtype, 
             if (!capturing && (tiles || (prompt && !w->dw.wh))) {
                 ZG_HIP(hipStreamSynchronize(s));
                 if (tiles) ZG_HIP(zg::ensure_mfma_tiles(const_cast<zg_weight*>(w)->dw, s));
-                if (prompt) ZG_HIP(zg::ensure_f16_tiles(const_cast<zg_weight*>(w)->dw, s));
+                if (prompt) {
+                    // (short of memory: the kernels of a captured call without them, below)
+                    const hipError_t e = zg::ensure_f16_tiles(const_cast<zg_weight*>(w)->dw, s);
+                    if (e != hipErrorOutOfMemory) ZG_HIP(e);
+                }
             }
             const size_t need = zg::batched_scratch_bytes(m_rows, w->dw.K);
             if (ctx->actbuf.bytes < need) ZG_HIP(hipStreamSynchronize(s));

@@ -358,8 +358,11 @@ hipError_t ensure_f16_tiles(DeviceWeight& w, hipStream_t s) {
     if (w.wh) return hipSuccess;
     const size_t tiles = (w.N + 31) / 32;
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, tiles * w.K * 64);
-    if (e != hipSuccess) return e;
+    hipError_t e = hipMalloc(&p, f16_tile_bytes(w.N, w.K));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // (the caller may go on without)
+        return e;
+    }
     hipLaunchKernelGGL(f16_tile_q4k_kernel, dim3((unsigned)tiles, (unsigned)(w.K / 256)), dim3(256), 0, s,
                        (const uint8_t*)w.qs, (const v4u*)w.hdr, (int)w.N, (int)w.K, (_Float16*)p);
     e = hipGetLastError();

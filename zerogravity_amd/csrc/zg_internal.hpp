@@ -286,9 +286,10 @@ size_t batched_scratch_bytes(size_t M, size_t K);
 // stream, so call it outside graph capture.  batched_gemv refuses a Q4_K
 // weight without them.
 hipError_t ensure_mfma_tiles(DeviceWeight& w, hipStream_t s);
-// Builds w.wh (Q4_K) if absent, likewise: batched_gemv refuses a prompt
-// (M >= kGemmRows) without it.
+// Builds w.wh (Q4_K) if absent, likewise.  Without it (hipErrorOutOfMemory:
+// nothing changed) a prompt (M >= kGemmRows) takes the 32-row kernel.
 hipError_t ensure_f16_tiles(DeviceWeight& w, hipStream_t s);
+inline size_t f16_tile_bytes(size_t N, size_t K) { return (N + 31) / 32 * K * 64; }
 hipError_t batched_gemv(const DeviceWeight& w, const FusedGemvArgs& a, void* scratch, hipStream_t s);
 // Q8_0 beyond 4 rows (zg_q8rows.hip): every activation row coded once into
 // `scratch` in act_prepare_for's layout (prepared_bytes(kQ8_0, M, K), within

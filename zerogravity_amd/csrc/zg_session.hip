@@ -1271,12 +1271,6 @@ int prefill_batched_body(zg_session* s, size_t row, size_t n, const uint32_t* to
     // them, and must find every other row as the host has it)
     int rc0 = sync_positions(s, st);
     if (rc0) return rc0;
-    // (the 32-row tiles at any length: the allocation-free call, which takes
-    // fewer rows, finds them after a prefill)
-    for (zg_weight* w : ws) {
-        if (!zg::xh16_layout(1, w->dw.K)) ZG_HIP(zg::ensure_mfma_tiles(w->dw, st));
-        if (n >= (size_t)zg::kGemmRows) ZG_HIP(zg::ensure_f16_tiles(w->dw, st));
-    }
     const size_t H = g.hidden, F = g.ffn, W = (size_t)g.gdn_heads * g.gdn_dim, GH = g.gdn_heads;
     const size_t QD = (size_t)g.q_heads * g.head_dim;
     const size_t mpad = (n + 31) / 32 * 32;
@@ -1302,6 +1296,23 @@ int prefill_batched_body(zg_session* s, size_t row, size_t n, const uint32_t* to
             ZG_HIP(hipMemsetAsync(s->pf[i], 0, std::max<size_t>(bytes[i], 256), st));  // stream-ordered
         }
         s->pf_cap = n;
+    }
+    // The weights' layouts, after the buffers.  The 32-row tiles at any length
+    // (the allocation-free call, which takes fewer rows, finds them after a
+    // prefill); for a long prompt the f16 tiles, or the 32-row ones, a quarter
+    // of their size, where memory is short of all that are missing.
+    size_t f16 = 0, room = 0, all = 0;
+    if (n >= (size_t)zg::kGemmRows) {
+        for (zg_weight* w : ws)
+            if (!w->dw.wh) f16 += zg::f16_tile_bytes(w->dw.N, w->dw.K);
+        if (f16) ZG_HIP(hipMemGetInfo(&room, &all));
+    }
+    for (zg_weight* w : ws) {
+        hipError_t e = hipErrorOutOfMemory;
+        if (n >= (size_t)zg::kGemmRows && (w->dw.wh || f16 <= room)) e = zg::ensure_f16_tiles(w->dw, st);
+        if (e != hipErrorOutOfMemory) ZG_HIP(e);
+        const bool rows32 = n >= (size_t)zg::kGemmRows && e == hipErrorOutOfMemory;
+        if (rows32 || !zg::xh16_layout(1, w->dw.K)) ZG_HIP(zg::ensure_mfma_tiles(w->dw, st));
     }
     float* x = (float*)s->pf[X];
     float* pj = (float*)s->pf[P];
