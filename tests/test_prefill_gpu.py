@@ -195,7 +195,7 @@ def test_prefill_batched_repeatable_and_tracks_token_prefill(kern):
     m.close()
 
 
-@pytest.mark.parametrize("n", [400, 600, 2048])
+@pytest.mark.parametrize("n", [256, 400, 600, 2048])
 def test_prefill_batched_prompt_gemm_matches_oracle(kern, n):
     """From 256 prompt rows every projection runs through the register-
     blocked prompt GEMM (zg_gemm.hip: Q4_K dequantized in registers, f16
@@ -228,6 +228,96 @@ def test_prefill_batched_prompt_gemm_matches_oracle(kern, n):
         assert e_state <= 1e-2
         tok = int(np.argmax(ref))
         assert int(np.argmax(s.forward(tok))) == int(np.argmax(o.forward(tok)))
+    m.close()
+
+
+LOUD = 7  # a token of its own, in the tests below
+
+
+def _loud_model(value, names):
+    """A 2B-shaped model in which the token LOUD alone drives the projections
+    `names` of the first layer to about 700 * value: its embedding, large, lies
+    in the first 256 columns, where their rows hold the constant `value`; for
+    the other tokens that block adds 16 * value on average."""
+    t = qwen35.synthetic_tensors(WIDE, gguf.Q4_K, seed=8)
+
+    def constant(blocks, value):
+        blocks[:, 0:2] = np.full(len(blocks), value, np.float16).view(np.uint8).reshape(-1, 2)
+        blocks[:, 2:4], blocks[:, 4:16], blocks[:, 16:] = 0, [1, 1, 1, 1, 0, 0, 0, 0, 1, 1, 1, 1], 0x11
+
+    for name, (codec, k, rows, data) in list(t.items()):
+        if name != "token_embd.weight" and name.split(".")[-2] not in names:
+            continue
+        b = np.array(data).reshape(rows, k // 256, 144)
+        if name == "token_embd.weight":
+            b[LOUD, :, :4] = 0  # zero but for the first block
+            constant(b[LOUD, :1], 100.0)
+        else:
+            constant(b[:, 0], value)
+        t[name] = (codec, k, rows, b.reshape(-1))
+    return t
+
+
+def _quiet(seed, n):
+    toks = _tokens(seed, n, WIDE["vocab"])
+    return np.where(toks == LOUD, LOUD + 1, toks).astype(np.uint32)
+
+
+def test_prompt_swiglu_of_large_gates_matches_oracle(kern):
+    """Gates past 80, where the prompt GEMM's SwiGLU takes its general form,
+    beside small ones in the same tiles."""
+    t = _loud_model(0.2, ["ffn_gate"])
+    m = qwen35.QwenModelHip(WIDE, t, kernel=kern)
+    s = m.session(max_batch=1, max_context=272, kv_dtype=L.BF16)
+    toks = _quiet(5, 256)
+    toks[[3, 40, 41, 200, 254]] = LOUD
+    lg, st = s.prefill_batched(toks), s.state()
+    with O.libm_mode(O.LIBM_GLIBC):
+        o = O.Model(WIDE, t).session(kv_bf16=True)
+        ref = _oracle_prefill(o, toks)
+        e_state = rel_err(st, o.state())
+    # (LOUD's own logit is a sum over its embedding, a hundred times the others')
+    lg, ref = np.delete(lg, LOUD), np.delete(ref, LOUD)
+    worst = float(np.max(np.abs(lg - ref)))
+    print(f"prompt SwiGLU of large gates: logits max-abs {worst:.3e} vs the oracle, state rel {e_state:.2e}")
+    assert worst <= LOGIT_TOL and int(np.argmax(lg)) == int(np.argmax(ref))
+    assert e_state <= 1e-2
+    m.close()
+
+
+def test_prompt_swiglu_of_a_token_does_not_depend_on_the_others(kern):
+    """The last token's gates, small or past 80, change no bit of an earlier
+    token's keys and values (layer 3's, after three SwiGLUs)."""
+    m = qwen35.QwenModelHip(WIDE, _loud_model(0.2, ["ffn_gate"]), kernel=kern)
+    s = m.session(max_batch=1, max_context=272, kv_dtype=L.F32)
+    n, got = 256, []
+    toks = _quiet(6, n)
+    for last in (LOUD, LOUD + 1):
+        toks[-1] = last
+        s.reset()
+        s.prefill_batched(toks)
+        kv = s.state()[-2 * n * 512:].reshape(2, n, 512)
+        assert np.abs(kv).max() > 0
+        got.append(kv[:, :-1].copy())
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    m.close()
+
+
+def test_prompt_swiglu_past_the_f16_range_fails_and_rolls_back(kern):
+    """A product past 65504 fails a long prompt (infinite in f16, its layer
+    is nonfinite) and leaves the row as it was; the next prompt is not
+    affected."""
+    m = qwen35.QwenModelHip(WIDE, _loud_model(0.5, ["ffn_gate", "ffn_up"]), kernel=kern)
+    s = m.session(max_batch=1, max_context=272, kv_dtype=L.BF16)
+    toks = _quiet(7, 256)
+    want = s.prefill_batched(toks)
+    s.reset()
+    bad = toks.copy()
+    bad[100] = LOUD
+    with pytest.raises(L.ZgError) as e:
+        s.prefill_batched(bad)
+    assert e.value.code == L.E_STATE and s.positions() == [0]
+    assert np.array_equal(s.prefill_batched(toks).view(np.uint32), want.view(np.uint32))
     m.close()
 
 

@@ -27,9 +27,9 @@ def kern():
 
 
 # one tile and the 256-row threshold, M and N one past and one short of a
-# tile, three and four K splits and none, a whole chip of each shape
+# tile, two, three and four K splits and none, a whole chip of each shape
 @pytest.mark.parametrize("M,N,K", [(256, 31, 256), (257, 129, 768), (300, 127, 3072), (385, 260, 3328), (601, 2048, 6144),
-                                   (640, 1030, 3584), (511, 8224, 1024), (1025, 2049, 2048), (2048, 8224, 512),
+                                   (700, 2044, 3072), (640, 1030, 3584), (511, 8224, 1024), (1025, 2049, 2048), (2048, 8224, 512),
                                    (4100, 4097, 256)])
 @pytest.mark.parametrize("norm", [False, True])
 def test_prompt_gemm_matches_float64(kern, M, N, K, norm):

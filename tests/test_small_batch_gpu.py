@@ -7,7 +7,9 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
+import zg_oracle as O
 from zerogravity_amd import _lib as L
+from zerogravity_amd import gguf, qwen35
 from zerogravity_amd import regions as R
 from zerogravity_amd import synth
 
@@ -43,3 +45,31 @@ def test_small_batch_matches_float64(kern, N, K, M):
     assert err.abs().max().item() <= 6e-3 * rms
     assert bool((y[M] == 7.0).all())
     kern.release_source(720)
+
+
+# the residual and SwiGLU forms, which a session's step alone reaches: 8-row
+# tiles (hidden 1024, 2048) with the next projection's tiles and sums, 16-row
+# tiles (3072) without; 2, 6 and 10 waves in the down projection
+@pytest.mark.parametrize("hidden,ffn", [(1024, 3072), (2048, 5120), (3072, 1024)])
+@pytest.mark.parametrize("B", [2, 5, 8])
+def test_small_batch_steps_match_oracle(kern, hidden, ffn, B):
+    """Three steps of B rows of a four-layer model, each row against its own
+    oracle session: logits within 2e-2, the end-to-end bound of the f16
+    projections, and the same greedy token where the oracle's best two are
+    further apart than two logits within that bound can move (4e-2)."""
+    g = dict(hidden=hidden, layers=4, ffn=ffn, vocab=1000, gdn_heads=16, gdn_dim=128, q_heads=8, kv_heads=2,
+             head_dim=256, full_attention_interval=4, max_context=4096, eps=1e-6)
+    t = qwen35.synthetic_tensors(g, gguf.Q4_K, seed=31)
+    m = qwen35.QwenModelHip(g, t, kernel=kern)
+    s = m.session(max_batch=B, max_context=64, kv_dtype=L.F32)
+    toks = np.random.default_rng(B).integers(0, g["vocab"], (3, B)).astype(np.uint32)
+    got = [s.step(row)[0] for row in toks]
+    om = O.Model(g, t)
+    for b in range(B):
+        o = om.session()
+        for i in range(3):
+            ref = o.forward(int(toks[i, b]))
+            assert float(np.max(np.abs(got[i][b] - ref))) <= 2e-2, (b, i)
+            second, first = np.sort(ref)[-2:]
+            assert first - second <= 4e-2 or int(np.argmax(got[i][b])) == int(np.argmax(ref)), (b, i)
+    m.close()

@@ -50,6 +50,8 @@ __device__ __forceinline__ void copy_frag(const _Float16* strip, int bytes, int 
 // and one residual correction instead of the scaled division.  The 16 values
 // of a lane's tile in ggml_silu took about 50 VALU instructions each, 19 us
 // of the 2048 x 12288 projection's 124.
+// Over every |gate| < 80 the bits are those of up * ggml_silu(gate), but for
+// the sign of a zero gate's product, so a tile may take either form.
 __device__ __forceinline__ float silu_product(float g, float up) {
     const float x = 0.0f - g, r = __uint_as_float(0x4b400000u);
     const float z = fmaf(x, __uint_as_float(0x3fb8aa3bu), r), n = z - r;
