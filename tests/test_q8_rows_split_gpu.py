@@ -30,3 +30,9 @@ def test_row_pairs_bit_exact(N, K, M):
     assert np.array_equal(got[:M].view(np.uint32), ref.view(np.uint32))
     assert (got[M] == 3.0).all()
     kern.ctx.close()
+
+
+@pytest.mark.parametrize("N,K,M", [(4090, 3584, 64), (12280, 1056, 32), (12280, 1056, 64), (300, 8192, 64)])
+def test_rows_dealt_over_rounds_bit_exact(N, K, M):
+    """Several workgroup rows, in one round of 512 workgroups and in more."""
+    test_row_pairs_bit_exact(N, K, M)

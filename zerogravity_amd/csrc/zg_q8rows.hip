@@ -405,23 +405,32 @@ hipError_t launch_mfma_rows(const FusedGemvArgs& a, const int8_t* aq, const floa
     // two workgroups per CU are all that its registers hold: more only stage
     // the activations again (151936 x 2048, 11 rows: 512 workgroups 105 us, 1024 116)
     const unsigned wgs = (unsigned)std::min<size_t>(((tiles + R - 1) / R + 3) / 4, 512);
-    // Activation rows per workgroup: at most 16 within 64 KB of LDS (two
-    // workgroups per CU), the rows dealt evenly over as few workgroup rows as
-    // that allows -- more when the tiles alone would leave CUs idle (each
-    // re-reads the weights from cache) -- and rounded up to whole pairs: the
-    // padding rows cost what real ones do.  151936 x 2048 head, us: 11 rows
-    // as 16 134, as 12 114; 17 rows as 16 + 16 252, as 10 + 10 192; 33 rows
-    // 366, as 3 x 12 306.
+    // Activation rows per workgroup: at most 16 within 64 KB of LDS, the rows
+    // dealt evenly over gy workgroup rows and rounded up to whole pairs (the
+    // padding rows cost what real ones do).  A round of 512 workgroups takes
+    // the time of its rows and of about 7 more for the loads, the staging and
+    // the finish; 256 and fewer, one to a CU, 0.87 of that.  gy is what comes
+    // out least.  Rows as gy x rows, us: head 151936 x 2048, 11 rows as 1 x 16
+    // 134, 1 x 12 114; 17 as 2 x 16 252, 2 x 10 192; 33 as 3 x 16 366, 3 x 12
+    // 306.  4096 x 3584, 64 rows as 5 x 14 (320 workgroups) 52.2, 8 x 8 (512)
+    // 36.2; 48 as 4 x 12 40.8, 8 x 6 31.8.  12288 x 3584, 17 rows as 3 x 6
+    // (576) 52.9, 2 x 10 (384) 43.3; 32 as 3 x 12 (576) 78.3, 4 x 8 (768) 62.8,
+    // 8 x 4 (1536) 77.9.
     int cap = 16;
     while (cap > 4 && rows_lds(cap, K) > 65536) cap -= 2;
-    int gy = (M + cap - 1) / cap;
-    while ((size_t)wgs * gy < 256 && (M + gy - 1) / gy > 4) ++gy;
+    if (rows_lds(cap, K) > 65536) return hipErrorInvalidValue;
     auto rows_of = [&](int y) { return std::max(4, ((M + y - 1) / y + 1) & ~1); };
-    // one workgroup row more where that pads less (16 rows as 4 x 4, not 3 x 6)
-    if ((size_t)wgs * gy < 512 && rows_of(gy) > 4 && rows_of(gy + 1) * (gy + 1) < rows_of(gy) * gy) ++gy;
+    auto cost = [&](int y) {
+        const long n = (long)wgs * y, rest = n % 512;
+        return (n / 512 * 100 + (rest > 256 ? 100 : rest > 0 ? 87 : 0)) * (rows_of(y) + 7);
+    };
+    const int least = (M + cap - 1) / cap, most = std::min((M + 3) / 4, least + 16);
+    int gy = least;
+    for (int y = least + 1; y <= most; ++y)
+        if (cost(y) * 1000 < cost(gy) * 975) gy = y;  // (more workgroup rows for 2.5% or more)
     const int mt = rows_of(gy);
     gy = (M + mt - 1) / mt;
-    if (rows_lds(mt, K) > 65536 || gy > 65535) return hipErrorInvalidValue;
+    if (gy > 65535) return hipErrorInvalidValue;
     const dim3 g(wgs, (unsigned)gy);
     const size_t lds = rows_lds(mt, K);
 #define ZG_Q8M(MP_, R_) hipLaunchKernelGGL((q8_mfma_kernel<MP_, R_, EPI>), g, dim3(256), lds, s, a, aq, ad)
