@@ -24,7 +24,7 @@ def kern():
 
 
 @pytest.mark.parametrize("N,K", [(8, 1024), (1001, 1024), (2040, 2048), (2048, 6144), (2049, 2048), (2064, 3072),
-                                 (333, 4096), (4100, 5120), (33001, 1024)])
+                                 (333, 4096), (4096, 5120), (4100, 5120), (8190, 3072), (33001, 1024)])
 @pytest.mark.parametrize("M", [2, 3, 7, 8, 9])
 def test_small_batch_matches_float64(kern, N, K, M):
     rng = np.random.default_rng(N + K + M)

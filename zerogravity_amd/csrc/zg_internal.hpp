@@ -262,7 +262,7 @@ int batched_splits(size_t N, size_t K);
 // (no split-K; xh16_layout(M, K) holds, and a residual projection with
 // rms_tiles_out leaves rms_ss_out[m][N/16]).
 bool batched16_supported(size_t M, size_t K, size_t N, int epi);
-// 2..8 rows of such a shape take the small-batch kernel (zg_small_batch.hip).
+// Whether 2..8 rows of such a shape take the small-batch kernel (zg_small_batch.hip).
 bool small_batch_fits(size_t M, size_t K, size_t N, int epi);
 hipError_t launch_small_batch(const FusedGemvArgs& a, const void* xh, hipStream_t s);
 // Columns per sum of squares a batched residual projection of this shape

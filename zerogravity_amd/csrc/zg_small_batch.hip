@@ -219,8 +219,15 @@ __global__ __launch_bounds__(64 * W) void small_batch_q4k_kernel(FusedGemvArgs a
 // 8-row tiles where 16-row ones would leave CUs without a workgroup.
 static int tile_rows(size_t N, int epi) { return epi != EPI_GLU && N <= 2048 && N % 8 == 0 ? 8 : 16; }
 
+// A CU holds 16 of the kernel's waves, of which 6, 10 or 12 to a workgroup
+// leave some empty: beyond one round of those, mfma16_q4k_kernel (8 waves).
+// At 3 rows, us, there against here: 16384 x 3072 13.7, 15.6; 8224 x 5120
+// 15.1, 16.1; 8224 x 6144 16.0, 17.1; within a round 4096 x 5120 11.1, 10.6,
+// 4096 x 6144 12.5, 11.2.
 bool small_batch_fits(size_t M, size_t K, size_t N, int epi) {
-    return M <= 8 && batched16_supported(M, K, N, epi) && (epi != EPI_GLU || (N / 2) % 8 == 0);
+    if (M > 8 || !batched16_supported(M, K, N, epi) || (epi == EPI_GLU && (N / 2) % 8)) return false;
+    const size_t W = K / 512, tr = tile_rows(N, epi), tiles = epi == EPI_GLU ? N / 16 : (N + tr - 1) / tr;
+    return 16 % W == 0 || tiles <= 256 * (16 / W);
 }
 
 int rms_ss_columns(size_t M, size_t K, size_t N) {
