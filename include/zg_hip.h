@@ -391,10 +391,12 @@ int zg_prefill(zg_session* s, size_t rows, size_t n, const uint32_t* tokens, flo
  * needs Q4_K projections (ZG_E_UNSUPPORTED otherwise).  Atomic: a failure
  * leaves the row's published state as it was, and the other rows' state and
  * positions untouched.  ZG_E_LIMIT when an operand of the prompt's
- * projections would reach 4 GiB (32-bit offsets: 32-row f16 activation
- * tiles of n x K, e.g. n >= 349,526 at K = 6144), or when the chunked GDN
- * prefill's output would (zg_gdn_chunk_prefill_device); split such a
- * prompt over several calls. */
+ * projections would reach 4 GiB (the f16 activation tiles of n x K, e.g.
+ * n >= 349,526 at K = 6144), or when the chunked GDN prefill's output would
+ * (zg_gdn_chunk_prefill_device); split such a prompt over several calls.
+ * The first call of 256 tokens or more lays the projections' weights out in
+ * f16 (2 bytes per weight, kept with them); where memory is short of that, it
+ * runs on a layout of a quarter of the size, slower. */
 int zg_prefill_batched(zg_session* s, size_t row, size_t n, const uint32_t* tokens, float* logits);
 /* Device-side step: d_tokens/d_logits/d_greedy are device pointers, no host
  * synchronisation.  The step's last kernel publishes it only if the status
@@ -448,8 +450,12 @@ int zg_session_fill_random(zg_session* s, size_t rows, size_t prefix, uint64_t s
  * bit-identical to the CPU at any M; Q4_K for one row, on the int8 matrix
  * cores; Q8_0 and Q6_K beyond 4 rows code each activation row once and
  * stream the weights once per 16 rows), and for Q4_K with M >= 2 the activation rounded to f16 and an f16
- * MFMA GEMM (f32 accumulate; within 1e-3 relative of the CPU), LDS-staged
- * for prompt-sized M >= 1024.
+ * MFMA GEMM (f32 accumulate; within 1e-3 relative of the CPU), for
+ * prompt-sized M >= 256 with the weight laid out once in f16 (2 bytes per
+ * weight).  The first call of a shape outside a graph capture lays the weight
+ * out and waits for it; a captured call runs on the layouts that are there,
+ * slower where a prompt's is not, and keeps the context's buffers only as
+ * long as no later call needs a larger activation.
  * No counterpart in the reference beyond MatVecKernel::try_execute; this is
  * the resident form the whole-program provider uses. */
 int zg_gemv_device(zg_ctx* ctx, const zg_weight* w, const void* x, int x_dtype, size_t m_rows,

@@ -613,7 +613,13 @@ constexpr int kSplitMaxChunks = 256;
 // chain is short, and at a 2k context one row gets one 32-token tile per
 // workgroup), about 512 beyond (two per CU: a workgroup's prologue -- the
 // q/k norms and RoPE -- costs more than a longer span); never more than
-// kSplitMaxChunks spans.
+// kSplitMaxChunks spans.  The rounding can leave a few more than the 512 that
+// run at once (24 rows of 1024: 528).  A 32-token longer span there gains only
+// while nearly every row fills its capacity, and costs otherwise: 24 x 1024
+// full 24.1 -> 20.3 us, three quarters full 19.1 -> 19.8, half 17.7 -> 19.5,
+// a quarter 16.6 -> 19.4; over 35 such shapes, geometric means 0.83, 1.04,
+// 1.05 and 1.06.  Sessions are sized for the longest request, so the span
+// stays.
 int attn_split_span(size_t B, int nkv, size_t max_ctx) {
     const size_t target = B <= 4 ? 256 : 512;
     const size_t want = (max_ctx * B * (size_t)nkv + target - 1) / target;

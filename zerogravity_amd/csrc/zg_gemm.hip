@@ -378,9 +378,11 @@ hipError_t ensure_f16_tiles(DeviceWeight& w, hipStream_t s) {
     return hipSuccess;
 }
 
-// Largest operand of the prompt GEMM in bytes: the f16 activation tiles (32
-// rows x K per tile) and the codec's own 32-row tiles and headers.  A prompt
-// at 4 GiB or more of any is refused.
+// What a prompt is refused by, at 4 GiB or more: the bytes of its f16
+// activation tiles (32 rows x K per tile) and of the weight's 32-row tiles and
+// headers.  No kernel needs the bound any more (offsets within a K strip, at
+// most 512 KB, are what is left in 32 bits); the f16 weight tiles, which it
+// does not count, may pass it.
 uint64_t prompt_gemm_bytes(size_t M, size_t K, size_t N) {
     const uint64_t mt = (M + 31) / 32, nt = (N + 31) / 32, nbk = K / 256;
     return std::max({mt * K * 64, nt * nbk * 4096, nt * nbk * 512});

@@ -1275,7 +1275,8 @@ int prefill_batched_body(zg_session* s, size_t row, size_t n, const uint32_t* to
     const size_t QD = (size_t)g.q_heads * g.head_dim;
     const size_t mpad = (n + 31) / 32 * 32;
     const size_t ldp = s->y0w;
-    // the prompt GEMM addresses each operand with 32-bit byte offsets
+    // (a limit of the call, kept from kernels with 32-bit byte offsets: the
+    // present ones address whole K strips from 64-bit pointers)
     for (zg_weight* w : ws)
         if (zg::prompt_gemm_bytes(n, w->dw.K, w->dw.N) >= ((uint64_t)1 << 32))
             return fail(ctx, ZG_E_LIMIT, "prompt too long for the batched prefill (an operand of its projections "
